@@ -102,19 +102,19 @@ __device__ __forceinline__ Mat<R, NC> staple_c(const Links<R, NC, COMP> &f, cons
 // sequence restoreSUN(U r1), restoreSUN(U r2), ... but a wave pays for that
 // work once per link instead of at every hit where any of its 64 lanes
 // accepts (about half the hits at 1 % acceptance).
-// accept iff dS < 0 or u < e^{-dS} (Metropolis.hpp:96-105)
+// accept iff dS < 0 or u < e^{-dS} (Metropolis.hpp:96-105).  e^{-dS} is first
+// taken from the FP32 exponential: its argument's rounding leaves a relative
+// error below dS 2^-22, under 2e-5 for the dS up to 87 whose result FP32 still
+// holds, so a u outside a 1e-4 band around it is decided as u < exp(-dS)
+// decides it.  Inside the band (one hit in 10^4), at u = 0 where the FP32 value
+// is 0 too, and for NaN, exp itself decides.
 template <typename R>
 __device__ __forceinline__ bool metro_accept(R dS, R u) {
-  bool accept = dS < R(0);
-  if (!accept) {
-    // e^x > 1 + x + x^2/2 + x^3/6 for x > 0, so u * that cubic >= 1 means
-    // u > e^{-dS}: a rejection found without the exponential.  dS > 1/2
-    // keeps the margin (> 0.1 %) far above rounding, so the decision is
-    // always the one u < e^{-dS} gives.
-    const R p3 = R(1) + dS * (R(1) + dS * (R(0.5) + dS * (R(1) / R(6))));
-    if (!(dS > R(0.5) && u * p3 >= R(1))) accept = u < exp(-dS);
-  }
-  return accept;
+  if (dS < R(0)) return true;
+  const float e = __builtin_amdgcn_exp2f(-1.44269504f * (float)dS), uf = (float)u;
+  if (uf > 1.0001f * e) return false;
+  if (uf < 0.9999f * e) return true;
+  return u < exp(-dS);
 }
 
 template <typename R, int NC>
