@@ -603,11 +603,11 @@ __global__ __launch_bounds__(256) void k_plaquette_walk(Links<R, NC, COMP> f, Ge
   double v = 0.0;
   if (sp < Vs) {
     int x[ND];
-    long long r = sp;
+    uint32_t r = (uint32_t)sp;
 #pragma unroll
     for (int d = ND - 1; d >= 1; --d) {
-      x[d] = (int)(r % g.L[d]);
-      r /= g.L[d];
+      x[d] = (int)(r % (uint32_t)g.L[d]);
+      r /= (uint32_t)g.L[d];
     }
     const int t0 = seg * S;
 #pragma unroll 1
@@ -896,12 +896,12 @@ __global__ __launch_bounds__(512) void k_wilson(Links<R, NC, COMP> f, Geom g, in
   const bool valid = cl < ncolblk && col < ncol;
   int x[ND];
   {
-    long long r = valid ? col : 0;
+    uint32_t r = valid ? (uint32_t)col : 0u;
 #pragma unroll
     for (int d = ND - 1; d >= 0; --d) {
       if (d == nu) continue;
-      x[d] = (int)(r % g.L[d]);
-      r /= g.L[d];
+      x[d] = (int)(r % (uint32_t)g.L[d]);
+      r /= (uint32_t)g.L[d];
     }
     x[nu] = k;
   }
