@@ -337,7 +337,7 @@ extern "C" int klft_field_create(int nd, int nc, const int *dims, int storage, k
   }
   f->max_partials = std::max<long long>(ki::kMinPartials, kd::link_blocks<4>(f->g) + 64);
   const size_t pbytes = ((sizeof(double) * (size_t)f->max_partials + 255) / 256) * 256;
-  size_t ws = pbytes + 256 + 16 * sizeof(double) + 8 * sizeof(unsigned long long);
+  size_t ws = pbytes + 256 + 16 * sizeof(double) + ki::kCounterRows * ki::kCounterCols * sizeof(unsigned long long);
   char *w = nullptr;
   e = hipMalloc((void **)&w, ws);
   if (e != hipSuccess) {

@@ -305,10 +305,11 @@ __device__ __forceinline__ void complete_row1(Mat<R, 2>& a) {
 // SU(3) FP64 sweep at nHits = 10 went from 0.96 to 0.82 ms on 16^4 and from
 // 1.86 to 1.68 ms on 32^4.
 __device__ __forceinline__ double inv_sqrt(double x) {
-  if (__builtin_expect(!(x > 0x1p-900 && x < 0x1p900), 0)) return 1.0 / sqrt(x);
   const double y = __builtin_amdgcn_rsq(x);
   const double e = fma(-(x * y), y, 1.0);
-  return fma(y * e, fma(e, 0.375, 0.5), y);
+  double r = fma(y * e, fma(e, 0.375, 0.5), y);
+  if (!((x > 0x1p-900) & (x < 0x1p900))) r = 1.0 / sqrt(x);
+  return r;
 }
 
 // restoreSUN<1,2,3>, the reference's (SUN.hpp:256-340) with its divisions by a
@@ -1002,31 +1003,30 @@ __device__ __forceinline__ bool row_scale(double n2, double& f) {
   f = inv_sqrt(n2);
   return true;
 }
-__device__ __forceinline__ bool rand_sun_w(const uint32_t* w, double delta, Mat<double, 3>& r) {
-  double v[6], fact;
-  cx<double> z1[3], z2[3];
+// six uniforms of [0, delta) as a row of three complex numbers of unit norm
+__device__ __forceinline__ bool unit_row_w(const uint32_t* w, double delta, cx<double>* z) {
+  double v[6], f;
 #pragma unroll
   for (int i = 0; i < 6; ++i) v[i] = draw_at<double>(w, i, 0.0, delta);
-  if (!row_scale(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3] + v[4] * v[4] + v[5] * v[5], fact)) return false;
+  if (!row_scale(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3] + v[4] * v[4] + v[5] * v[5], f)) return false;
 #pragma unroll
-  for (int i = 0; i < 3; ++i) z1[i] = mk(fact * v[2 * i], fact * v[2 * i + 1]);
-#pragma unroll
-  for (int i = 0; i < 6; ++i) v[i] = draw_at<double>(w, 6 + i, 0.0, delta);
-  if (!row_scale(v[0] * v[0] + v[1] * v[1] + v[2] * v[2] + v[3] * v[3] + v[4] * v[4] + v[5] * v[5], fact)) return false;
-#pragma unroll
-  for (int i = 0; i < 3; ++i) z2[i] = mk(fact * v[2 * i], fact * v[2 * i + 1]);
+  for (int i = 0; i < 3; ++i) z[i] = mk(f * v[2 * i], f * v[2 * i + 1]);
+  return true;
+}
+// the rows r_0, r_1 orthonormalised, the third completed
+__device__ __forceinline__ bool unitary_rows(const cx<double>* z1, cx<double>* z2, Mat<double, 3>& r) {
   const cx<double> z = cmul_(z1[0], z2[0]) + cmul_(z1[1], z2[1]) + cmul_(z1[2], z2[2]);
 #pragma unroll
   for (int i = 0; i < 3; ++i) z2[i] = z2[i] - z * z1[i];
+  double f;
   if (!row_scale(z2[0].re * z2[0].re + z2[0].im * z2[0].im + z2[1].re * z2[1].re + z2[1].im * z2[1].im +
                      z2[2].re * z2[2].re + z2[2].im * z2[2].im,
-                 fact))
+                 f))
     return false;
 #pragma unroll
   for (int i = 0; i < 3; ++i) {
-    z2[i] = scale(fact, z2[i]);
     r.m[0][i] = z1[i];
-    r.m[1][i] = z2[i];
+    r.m[1][i] = scale(f, z2[i]);
   }
   complete_row2(r);
   return true;
@@ -1036,14 +1036,39 @@ __device__ __forceinline__ bool rand_sun_w(const uint32_t* w, double delta, Mat<
 template <typename R, int NC>
 __device__ __forceinline__ void propose(uint64_t seed, uint32_t site, uint32_t sweep, uint32_t hit,
                                         uint32_t chain, uint32_t mu, R delta, Mat<R, NC>& r, R& u) {
-  constexpr int NB = (HitDraws<NC>::value * DrawWords<R>::value + 3) / 4;
   const klft_rng::Stream st(seed, klft_rng::TAG_METROPOLIS, site, sweep, hit, chain, mu);
-  uint32_t w[4 * NB];
+  if constexpr (sizeof(R) == 8 && NC == 3) {
+    // Row by row: a row takes the stream's next three blocks (12 words) and is
+    // drawn again from the three after them when it is rejected, the rejection
+    // loops of SUN.hpp:198-233.  All seven blocks of the usual case at once,
+    // with the looping rand_sun as a second path, hold 220 registers, this 100.
+    uint32_t w[16], j = 0;
+    cx<double> z1[3], z2[3];
+    bool ok;
+    do {
 #pragma unroll
-  for (int j = 0; j < NB; ++j) st.block_words((uint32_t)j, w + 4 * j);
-  if (rand_sun_w(w, delta, r)) {
-    u = u01_at<R>(w, HitDraws<NC>::value - 1);
+      for (uint32_t k = 0; k < 3; ++k) st.block_words(j + k, w + 4 * k);
+      ok = unit_row_w(w, delta, z1);
+      j += 3;
+    } while (!ok);
+    do {
+      // the block after the row's holds the accept uniform
+#pragma unroll
+      for (uint32_t k = 0; k < 4; ++k) st.block_words(j + k, w + 4 * k);
+      ok = unit_row_w(w, delta, z2) && unitary_rows(z1, z2, r);
+      j += 3;
+    } while (!ok);
+    u = u01_at<R>(w, 6);
     return;
+  } else {
+    constexpr int NB = (HitDraws<NC>::value * DrawWords<R>::value + 3) / 4;
+    uint32_t w[4 * NB];
+#pragma unroll
+    for (int j = 0; j < NB; ++j) st.block_words((uint32_t)j, w + 4 * j);
+    if (rand_sun_w(w, delta, r)) {
+      u = u01_at<R>(w, HitDraws<NC>::value - 1);
+      return;
+    }
   }
   klft_rng::Stream s2 = st;
   rand_sun(s2, delta, r);

@@ -29,12 +29,12 @@ struct klft_field_s {
   long long max_partials = 0;  // capacity of partials: the largest reduction grid
   unsigned int *ticket = nullptr;
   double *result = nullptr;  // 16 doubles
-  unsigned long long *counter = nullptr;  // 8 counters
+  unsigned long long *counter = nullptr;  // kCounterRows rows of kCounterCols counters
   double *host_result = nullptr;          // pinned, 16 doubles
-  // per-sweep acceptance counters of klft_metropolis_run (grown on demand,
-  // kept until the field is destroyed)
+  // acceptance counters of klft_metropolis_run, kCounterRows rows of one per
+  // sweep (grown on demand, kept until the field is destroyed)
   unsigned long long *run_counters = nullptr;
-  int run_capacity = 0;
+  long long run_capacity = 0;
   // measurement workspace (Wilson-loop partials, outputs, extents; grown on
   // demand, kept until the field is destroyed)
   void *meas_ws = nullptr;
@@ -47,6 +47,18 @@ namespace klft_internal {
 // reduction partials per field: at least this many, and at least one per
 // block of the largest grid (one thread per link, 64 sites per block)
 constexpr long long kMinPartials = 1 << 16;
+
+// Acceptance counters.  An atomic add to one address takes about 10 ns on this
+// GPU (it is served at the memory side, across the XCDs' L2s), so the blocks of
+// a launch spread theirs over kCounterRows rows, blocks b of equal
+// b % kCounterRows sharing one; a sweep's count is the sum of its column.
+constexpr int kCounterRows = 16;
+constexpr int kCounterCols = 16;  // of a field's fixed counters: one line per row
+struct Counters {
+  unsigned long long *base;
+  int per_sweep;  // columns from one sweep of a run to the next
+  int row;        // row length
+};
 
 int set_error(int code, const char *fmt, ...);
 int ensure_init();
@@ -71,7 +83,7 @@ int enqueue_reunit(klft_field_t f);
 // that wrote them)
 int enqueue_sum_blocks(const double *partials, long long n, double *out);
 int enqueue_sweep(klft_field_t f, const klft_metropolis_params *p, uint64_t sweep, uint32_t chain,
-                  unsigned long long *counter, int *visit);
+                  Counters counter, int *visit);
 int check_field(const klft_field_s *f);
 int sync_stream();
 

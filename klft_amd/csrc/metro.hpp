@@ -110,11 +110,11 @@ __device__ __forceinline__ Mat<R, NC> staple_c(const Links<R, NC, COMP> &f, cons
 // is 0 too, and for NaN, exp itself decides.
 template <typename R>
 __device__ __forceinline__ bool metro_accept(R dS, R u) {
-  if (dS < R(0)) return true;
   const float e = __builtin_amdgcn_exp2f(-1.44269504f * (float)dS), uf = (float)u;
-  if (uf > 1.0001f * e) return false;
-  if (uf < 0.9999f * e) return true;
-  return u < exp(-dS);
+  // no short-circuit: one branch, to the band
+  bool acc = (dS < R(0)) | (uf < 0.9999f * e);
+  if (!(acc | (uf > 1.0001f * e))) acc = u < exp(-dS);
+  return acc;
 }
 
 template <typename R, int NC>

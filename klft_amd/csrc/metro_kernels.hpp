@@ -1,7 +1,5 @@
-// Checkerboarded Metropolis sweep kernels (Metropolis.hpp:44-178) and their
-// launcher, instantiated per link storage in metropolis_f64.hip,
-// metropolis_f32.hip and metropolis_f32rows.hip (the three translation units
-// compile in parallel).  The algorithm is described in metropolis.hip.
+// Checkerboarded Metropolis sweep kernels (Metropolis.hpp:44-178), launched by
+// metro_launch.hpp.  The algorithm is described in metropolis.hip.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -413,7 +411,7 @@ template <typename R, int NC, bool COMP, int ND, bool ILV, bool SYM = false>
 __global__ __launch_bounds__(kWsBlock, (sizeof(R) == 4 && !ILV) ? 4 : 2) void k_metropolis_ws(
     Links<R, NC, COMP> f, Geom g, int pass, int pass2, int nhits, R beta_nc, R delta, uint64_t seed,
     uint32_t sweep, uint32_t sweep2, uint32_t chain, unsigned long long *nacc, unsigned long long *nacc2,
-    int *visit) {
+    int nacc_row, int *visit) {
   f.nd = ND;
   __shared__ cx<R> stage[4 * 4 * NC * NC * 64];
   __shared__ unsigned long long red[kWsBlock / 64];
@@ -430,117 +428,7 @@ __global__ __launch_bounds__(kWsBlock, (sizeof(R) == 4 && !ILV) ? 4 : 2) void k_
   const unsigned long long n = ws_pass<R, NC, COMP, ND, ILV, false, SYM>(f, g, pass, t, nhits, beta_nc, delta,
                                                                          seed, sweep, chain, visit, Defect{}, R(1),
                                                                          stage);
-  ws_count(n, red, nacc);
+  ws_count(n, red, nacc + (size_t)(blockIdx.x % kCounterRows) * nacc_row);
 }
-
-// Sweep variants (numbers kept stable for tuning caches): 0 one lane per
-// site; 4 one lane, low-register staple, >= 2 waves per SIMD; 7 one lane,
-// next direction's staple loaded during the hits; 11 one lane, the site's own
-// links kept in registers; 12 site waves fed by staple waves; 13 the same with
-// each direction's upper and lower staple terms back to back; 14, 15: 12, 13
-// with the symmetric SU(3) proposal.  1-3, 5, 6, 8-10 (four or two lanes per
-// site, proposals drawn in pairs, LDS-staged staple terms) never won at
-// 16^4 - 48^4 and were removed.
-template <typename RR, bool CC>
-int launch_passes_typed(klft_field_t f, void *links, int variant, int p0, int p1,
-                        const klft_metropolis_params *p, uint64_t sweep, int nsweeps, uint32_t chain,
-                        unsigned long long *counter, int counter_stride, int *visit) {
-  return dispatch_typed<RR, CC>(f->nc, f->nd, [&](auto rt, auto nct, auto ct, auto ndt) -> int {
-    KLFT_UNPACK(rt, nct, ct, ndt);
-    Links<R, NC, COMP> l;
-    l.p = reinterpret_cast<cx<R> *>(links);
-    l.V = f->g.V;
-    l.nd = f->nd;
-    const R beta_nc = (R)(p->beta / (double)NC);
-    const unsigned nb = blocks_for(f->g.Vh, kMetroBlock);
-    switch (variant) {
-      case 0: case 4: case 7: case 11: case 12: case 13: case 14: case 15: break;
-      default: return set_error(KLFT_E_ARG, "sweep variant %d is not built", variant);
-    }
-    // acceptance counter of sweep i of the run (relative to `sweep`)
-    auto cnt = [&](int i) { return counter + (long long)i * counter_stride; };
-    const unsigned nws = blocks_for(f->g.Vh, kWsSites);
-    // launch the site-wave kernel on one pass (pb < 0), or on two
-    // independent ones, each with its own sweep and counter
-    auto ws = [&](auto kern, int pa, int sa, int pb, int sb) {
-      hipLaunchKernelGGL(kern, dim3(pb >= 0 ? 2 * nws : nws), dim3(kWsBlock), 0, stream(), l, f->g, pa, pb,
-                         p->nhits, beta_nc, (R)p->delta, p->seed, (uint32_t)(sweep + sa), (uint32_t)(sweep + sb),
-                         chain, cnt(sa), cnt(sb), visit);
-    };
-    auto launch_ws = [&](int pa, int sa, int pb, int sb) -> int {
-      switch (variant) {
-        case 12: ws(k_metropolis_ws<R, NC, COMP, ND, false>, pa, sa, pb, sb); break;
-        case 13: ws(k_metropolis_ws<R, NC, COMP, ND, true>, pa, sa, pb, sb); break;
-        default:
-          // the symmetric SU(3) proposal: site waves, terms as in 12 / 13
-          if constexpr (NC == 3) {
-            if (variant == 14)
-              ws(k_metropolis_ws<R, NC, COMP, ND, false, true>, pa, sa, pb, sb);
-            else
-              ws(k_metropolis_ws<R, NC, COMP, ND, true, true>, pa, sa, pb, sb);
-          } else {
-            return set_error(KLFT_E_ARG, "the symmetric proposal variants are SU(3) only");
-          }
-      }
-      return KLFT_OK;
-    };
-    // whole sweeps run their independent passes in pairs when both passes'
-    // blocks fit on the GPU at once (KLFT_VARIANT=metropolis_pairs=0: never);
-    // a run of several sweeps also pairs passes of consecutive sweeps
-    // (run_schedule)
-    bool pair = false;
-    if (variant >= 12 && p0 == 0 && p1 == (1 << ND) && forced_variant("metropolis_pairs") != 0) {
-      const void *kern = nullptr;
-      switch (variant) {
-        case 12: kern = reinterpret_cast<const void *>(&k_metropolis_ws<R, NC, COMP, ND, false>); break;
-        case 13: kern = reinterpret_cast<const void *>(&k_metropolis_ws<R, NC, COMP, ND, true>); break;
-        case 14: kern = reinterpret_cast<const void *>(&k_metropolis_ws<R, NC, COMP, ND, false, true>); break;
-        default: kern = reinterpret_cast<const void *>(&k_metropolis_ws<R, NC, COMP, ND, true, true>); break;
-      }
-      pair = 2LL * nws <= (long long)cu_count() * blocks_per_cu(kern, kWsBlock);
-    }
-    if (pair) {
-      int rc = KLFT_OK;
-      for_each_run_launch(ND, nsweeps, [&](const RunLaunch &L) {
-        if (rc) return;
-        const int pa = L.pass[0], pb = L.pass[1];
-        char label[56];
-        if (pb >= 0)
-          snprintf(label, sizeof label, "sweep_Metropolis_GaugeField_sublat_%d_%d", pa, pb);
-        else
-          snprintf(label, sizeof label, "sweep_Metropolis_GaugeField_sublat_%d", pa);  // Metropolis.hpp:161
-        ProfScope prof(pb >= 0 ? "metropolis_pass_pair" : "metropolis_pass", label);
-        rc = launch_ws(pa, L.sweep[0], pb, pb >= 0 ? L.sweep[1] : L.sweep[0]);
-      });
-      if (rc) return rc;
-    } else {
-      for (int i = 0; i < nsweeps; ++i) {
-        for (int pass = p0; pass < p1; ++pass) {
-          char label[48];
-          snprintf(label, sizeof label, "sweep_Metropolis_GaugeField_sublat_%d", pass);  // Metropolis.hpp:161
-          ProfScope prof("metropolis_pass", label);
-          if (variant >= 12) {
-            const int rc = launch_ws(pass, i, -1, i);
-            if (rc) return rc;
-          } else {
-            auto one_lane = [&](auto kern) {
-              hipLaunchKernelGGL(kern, dim3(nb), dim3(kMetroBlock), 0, stream(), l, f->g, pass, p->nhits, beta_nc,
-                                 (R)p->delta, p->seed, (uint32_t)(sweep + i), chain, cnt(i), visit);
-            };
-            switch (variant) {
-              case 4: one_lane(k_metropolis_pass<R, NC, COMP, ND, true, 2>); break;
-              case 7: one_lane(k_metropolis_pipe<R, NC, COMP, ND>); break;
-              case 11: one_lane(k_metropolis_own<R, NC, COMP, ND>); break;
-              default: one_lane(k_metropolis_pass<R, NC, COMP, ND, false, 1>); break;
-            }
-          }
-        }
-      }
-    }
-    KLFT_HIP(hipGetLastError());
-    return KLFT_OK;
-  });
-}
-
 
 }  // namespace klft_metro

@@ -14,6 +14,7 @@
 // (M r and S restoreSUN(U r) differ by rounding only).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <string>
 #include <vector>
 
@@ -22,18 +23,16 @@
 using namespace kd;
 namespace ki = klft_internal;
 
-constexpr int kMetroVariants = 14;
+constexpr int kMetroVariants = 18;
 
 namespace klft_internal {
 int launch_passes_f64(klft_field_t f, void *links, int variant, int p0, int p1, const klft_metropolis_params *p,
-                      uint64_t sweep, int nsweeps, uint32_t chain, unsigned long long *counter,
-                      int counter_stride, int *visit);
+                      uint64_t sweep, int nsweeps, uint32_t chain, Counters counter, int *visit);
 int launch_passes_f32(klft_field_t f, void *links, int variant, int p0, int p1, const klft_metropolis_params *p,
-                      uint64_t sweep, int nsweeps, uint32_t chain, unsigned long long *counter,
-                      int counter_stride, int *visit);
+                      uint64_t sweep, int nsweeps, uint32_t chain, Counters counter, int *visit);
 int launch_passes_f32rows(klft_field_t f, void *links, int variant, int p0, int p1,
                           const klft_metropolis_params *p, uint64_t sweep, int nsweeps, uint32_t chain,
-                          unsigned long long *counter, int counter_stride, int *visit);
+                          Counters counter, int *visit);
 }  // namespace klft_internal
 
 __global__ void k_zero_u64(unsigned long long *p, int n) {
@@ -45,26 +44,45 @@ namespace klft_internal {
 
 // launch passes [p0, p1) of sweeps sweep .. sweep + nsweeps - 1 on the link
 // array `links`, sweep i counting its accepted hits into
-// counter[i * counter_stride]; the kernels are instantiated per storage in
+// column i * counter.per_sweep; the kernels are instantiated per storage in
 // metropolis_{f64,f32,f32rows}.hip (the variant table is in
 // metro_kernels.hpp).  U(1) has no compressed form, so its two-row storage
 // runs the FP32 kernels.
 static int launch_passes(klft_field_t f, void *links, int variant, int p0, int p1,
                          const klft_metropolis_params *p, uint64_t sweep, int nsweeps, uint32_t chain,
-                         unsigned long long *counter, int counter_stride, int *visit) {
+                         Counters counter, int *visit) {
   switch (f->storage) {
     case KLFT_STORAGE_F64:
-      return launch_passes_f64(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, counter_stride, visit);
+      return launch_passes_f64(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, visit);
     case KLFT_STORAGE_F32:
-      return launch_passes_f32(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, counter_stride, visit);
+      return launch_passes_f32(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, visit);
     case KLFT_STORAGE_F32_ROWS:
       if (f->nc == 1)
-        return launch_passes_f32(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, counter_stride,
-                                 visit);
-      return launch_passes_f32rows(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, counter_stride,
-                                   visit);
+        return launch_passes_f32(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, visit);
+      return launch_passes_f32rows(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter, visit);
   }
   return set_error(KLFT_E_ARG, "storage=%d unsupported", f->storage);
+}
+
+// Whether a pass of Vh sites runs faster with a link's hits in parallel
+// (metro_hits.hpp) than with site waves fed by staple waves.  The site-wave
+// kernel's pass costs one block's serial chain however few blocks there are;
+// the hit-parallel kernel's chain is four to six times shorter but spends up
+// to ten lanes on a site, so it wins until the sites fill the GPU.  Measured
+// ms per sweep in runs, nHits = 10, hit-parallel / site waves, around the
+// limits (sites of a pass per CU):
+//   SU(3)  16/CU (16^4) FP64 0.23 / 0.64, FP32 0.17 / 0.49; 81/CU (24^4) FP64
+//          0.68 / 0.71, FP32 0.44 / 0.50; with 1 hit 57/CU (22^4) 0.47 / 0.44
+//   SU(2)  16/CU FP64 0.32 / 0.52; 26/CU (18^4) 0.48 / 0.52, FP32 0.29 / 0.35;
+//          39/CU (20^4) 0.67 / 0.52
+//   U(1)   16/CU FP64 0.22 / 0.28; 26/CU 0.30 / 0.28, FP32 0.22 / 0.23; with 4
+//          hits 39/CU 0.16 / 0.19
+// and in 2D with fewer than 4 hits the site waves' chain is as short (U(1)
+// 32^2, 1 hit: 32 against 29 us).
+static bool hits_in_parallel(klft_field_t f, int nhits) {
+  if (f->nd == 2 && nhits < 4) return false;
+  const int per_cu = f->nc == 3 ? (nhits < 8 ? 48 : 81) : (f->nc == 2 ? 27 : (nhits < 5 ? 40 : 20));
+  return f->g.Vh <= (long long)per_cu * cu_count();
 }
 
 // sweep variant for this field; tuning times one sweep of each variant on a
@@ -73,62 +91,72 @@ static int launch_passes(klft_field_t f, void *links, int variant, int p0, int p
 // both fit on the GPU at once, which a single pass would not show)
 int metropolis_variant(klft_field_t f, const klft_metropolis_params *p, bool timed) {
   void *scratch = nullptr;
-  // variants (metro_kernels.hpp): 0 one lane per site; 4 one lane with the
+  // variants (metro_launch.hpp): 0 one lane per site; 4 one lane with the
   // low-register staple at >= 2 waves/SIMD; 7 one lane building the next
   // direction's staple during the hits; 11 one lane with the site's own links
-  // kept in registers; 12 site waves fed the next staple by staple waves; 13
-  // the same with each direction's upper and lower staple terms back to back.
-  // The other numbers below kMetroVariants are not built (the tuner skips
-  // them).
-  // Untuned defaults: site waves fed by staple waves, the fastest at 16^4,
-  // 24^4 and 32^4 for every group (nHits = 10), with the interleaved term
-  // order for FP64 links.  For FP32 links the interleaved order's six loads
-  // in flight (196 VGPRs) leave room for one block per CU, the
-  // upper-terms-first order (128 VGPRs) for two: the interleaved order wins
-  // while two paired passes fill at most one block per CU, and loses once
-  // they need two (32^4: two-block pairs) or blocks queue for a CU (48^4:
-  // 398 against 308 us per pass).
+  // kept in registers; 12 site waves fed by staple waves; 13 the same with
+  // each direction's upper and lower staple terms back to back; 16, 17 the
+  // hits of a link in parallel, staple terms summed as in 12, 13.  The other
+  // numbers below kMetroVariants are not built (the tuner skips them), or run
+  // the symmetric proposal (14, 15).
+  // Untuned defaults: hits in parallel while the sites do not fill the GPU
+  // (hits_in_parallel), else site waves fed by staple waves, with the
+  // interleaved term order for FP64 links.  For FP32 links the interleaved
+  // order's six loads in flight (196 VGPRs) leave room for one block per CU,
+  // the upper-terms-first order (128 VGPRs) for two: the interleaved order
+  // wins while two paired passes fill at most one block per CU, and loses once
+  // they need two (32^4: two-block pairs) or blocks queue for a CU (48^4: 398
+  // against 308 us per pass).  The order of the terms is a matter of the size
+  // alone, so that the FP32 results do not depend on which kernel runs.
   const bool paired_one_round = 2 * ((f->g.Vh + 255) / 256) <= (long long)cu_count();
-  const int dflt = (f->storage == KLFT_STORAGE_F64 || paired_one_round) ? 13 : 12;
-  // the symmetric SU(3) proposal runs in the site-wave kernels only
+  const int dflt = ((f->storage == KLFT_STORAGE_F64 || paired_one_round) ? 13 : 12) +
+                   (hits_in_parallel(f, p->nhits) ? 4 : 0);
+  // the symmetric SU(3) proposal runs in these kernels only
   if (f->proposal == KLFT_PROPOSAL_SYMMETRIC && f->nc == 3) return dflt + 2;
   // KLFT_VARIANT="metropolis=v" forces a variant for every hit count
+  auto reference_law = [](int v) { return v != 14 && v != 15; };
   const int fv = forced_variant("metropolis");
-  if (fv >= 0 && fv < kMetroVariants) return fv;
+  if (fv >= 0 && fv < kMetroVariants && reference_law(fv)) return fv;
   // the tuning key carries nHits: the best variant depends on the hit count
   const std::string kname = "metropolis_nhits_" + std::to_string(p->nhits);
-  if (!timed) return chosen_variant(kname.c_str(), f, kMetroVariants, dflt);
-  const int v = pick_variant(kname.c_str(), f, kMetroVariants, dflt, [&](int var) -> int {
-    if (!scratch) {
-      KLFT_HIP(hipMalloc(&scratch, f->link_bytes));
-      KLFT_HIP(hipMemcpyAsync(scratch, f->links, f->link_bytes, hipMemcpyDeviceToDevice, stream()));
+  int v;
+  if (!timed) {
+    v = chosen_variant(kname.c_str(), f, kMetroVariants, dflt);
+  } else {
+    v = pick_variant(kname.c_str(), f, kMetroVariants, dflt, [&](int var) -> int {
+      if (!reference_law(var)) return KLFT_E_ARG;
+      if (!scratch) {
+        KLFT_HIP(hipMalloc(&scratch, f->link_bytes));
+        KLFT_HIP(hipMemcpyAsync(scratch, f->links, f->link_bytes, hipMemcpyDeviceToDevice, stream()));
+      }
+      return launch_passes(f, scratch, var, 0, 1 << f->nd, p, 0, 1, 0, Counters{f->counter + 7, 0, kCounterCols},
+                           nullptr);
+    });
+    if (scratch) {
+      (void)hipStreamSynchronize(stream());
+      (void)hipFree(scratch);
     }
-    return launch_passes(f, scratch, var, 0, 1 << f->nd, p, 0, 1, 0, f->counter + 7, 0, nullptr);
-  });
-  if (scratch) {
-    (void)hipStreamSynchronize(stream());
-    (void)hipFree(scratch);
   }
-  return v;
+  return reference_law(v) ? v : dflt;
 }
 
-// enqueue one sweep (no synchronisation); acceptance counted into *counter
+// enqueue one sweep (no synchronisation); acceptance counted into `counter`
 int enqueue_sweep(klft_field_t f, const klft_metropolis_params *p, uint64_t sweep, uint32_t chain,
-                  unsigned long long *counter, int *visit) {
+                  Counters counter, int *visit) {
   // the schedule dump (visit != nullptr, nHits = 0) is never timed: its
   // staple-only passes are not the workload a tuned variant is chosen for
   const int v = metropolis_variant(f, p, visit == nullptr);
-  return launch_passes(f, f->links, v, 0, 1 << f->nd, p, sweep, 1, chain, counter, 0, visit);
+  return launch_passes(f, f->links, v, 0, 1 << f->nd, p, sweep, 1, chain, counter, visit);
 }
 
 // enqueue sweeps sweep0 .. sweep0 + n - 1 (no synchronisation), passes of
 // consecutive sweeps sharing launches where they are independent; sweep i
-// counts into counter[i * counter_stride]
+// counts into column i * counter.per_sweep
 static int enqueue_run(klft_field_t f, const klft_metropolis_params *p, uint64_t sweep0, int n,
-                       unsigned long long *counter, int counter_stride) {
+                       Counters counter) {
   if (n <= 0) return KLFT_OK;
   const int v = metropolis_variant(f, p, true);
-  return launch_passes(f, f->links, v, 0, 1 << f->nd, p, sweep0, n, 0, counter, counter_stride, nullptr);
+  return launch_passes(f, f->links, v, 0, 1 << f->nd, p, sweep0, n, 0, counter, nullptr);
 }
 
 }  // namespace klft_internal
@@ -154,12 +182,14 @@ extern "C" int klft_metropolis_sweep(klft_field_t f, const klft_metropolis_param
                                      double *acc_rate, int64_t *naccepted) {
   int rc = check_params(f, p);
   if (rc) return rc;
-  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, ki::stream(), f->counter, 1);
-  rc = ki::enqueue_sweep(f, p, sweep, 0, f->counter, nullptr);
+  constexpr int nc = ki::kCounterRows * ki::kCounterCols;
+  hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(nc), 0, ki::stream(), f->counter, nc);
+  rc = ki::enqueue_sweep(f, p, sweep, 0, ki::Counters{f->counter, 0, ki::kCounterCols}, nullptr);
   if (rc) return rc;
-  unsigned long long n = 0;
-  KLFT_HIP(hipMemcpyAsync(&n, f->counter, sizeof n, hipMemcpyDeviceToHost, ki::stream()));
+  unsigned long long h[nc], n = 0;
+  KLFT_HIP(hipMemcpyAsync(h, f->counter, sizeof h, hipMemcpyDeviceToHost, ki::stream()));
   KLFT_HIP(hipStreamSynchronize(ki::stream()));
+  for (int r = 0; r < ki::kCounterRows; ++r) n += h[r * ki::kCounterCols];
   if (naccepted) *naccepted = (int64_t)n;
   if (acc_rate) *acc_rate = acceptance(f, p->nhits, n);
   return KLFT_OK;
@@ -170,34 +200,44 @@ extern "C" int klft_metropolis_run(klft_field_t f, const klft_metropolis_params 
   int rc = check_params(f, p);
   if (rc) return rc;
   if (n < 0) return ki::set_error(KLFT_E_ARG, "negative sweep count");
-  unsigned long long *cnt = nullptr;
-  if (acc_rates && n > 0) {
-    // one counter per sweep, in a buffer kept with the field (grown only when
-    // a longer run asks for more) and cleared by a kernel
-    if (n > f->run_capacity) {
+  // one column of counters per sweep, in a buffer kept with the field (grown
+  // only when a longer run asks for more) and cleared by a kernel; rows of
+  // whole lines
+  const bool rates = acc_rates && n > 0;
+  ki::Counters cnt{f->counter, 0, ki::kCounterCols};
+  long long ncnt = (long long)ki::kCounterRows * ki::kCounterCols;
+  if (rates) {
+    if (n > (1 << 26)) return ki::set_error(KLFT_E_ARG, "at most 2^26 sweeps per run with rates");
+    cnt.row = (n + 15) / 16 * 16;
+    ncnt = (long long)ki::kCounterRows * cnt.row;
+    if (ncnt > f->run_capacity) {
       if (f->run_counters) {
         KLFT_HIP(hipStreamSynchronize(ki::stream()));
         (void)hipFree(f->run_counters);
         f->run_counters = nullptr;
         f->run_capacity = 0;
       }
-      const int cap = n > 1024 ? n : 1024;
+      const long long cap = std::max<long long>(ncnt, 1024 * ki::kCounterRows);
       KLFT_HIP(hipMalloc(&f->run_counters, sizeof(unsigned long long) * cap));
       f->run_capacity = cap;
     }
-    cnt = f->run_counters;
-    hipLaunchKernelGGL(k_zero_u64, dim3(ki::blocks_for(n, 256)), dim3(256), 0, ki::stream(), cnt, n);
-  } else {
-    hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(64), 0, ki::stream(), f->counter, 1);
+    cnt.base = f->run_counters;
+    cnt.per_sweep = 1;
   }
-  rc = ki::enqueue_run(f, p, sweep0, n, cnt ? cnt : f->counter, cnt ? 1 : 0);
-  if (!rc && cnt) {
-    std::vector<unsigned long long> h(n);
-    hipError_t e = hipMemcpyAsync(h.data(), cnt, sizeof(unsigned long long) * n, hipMemcpyDeviceToHost,
+  hipLaunchKernelGGL(k_zero_u64, dim3((unsigned)std::min<long long>((ncnt + 255) / 256, 4096)), dim3(256), 0,
+                     ki::stream(), cnt.base, (int)ncnt);
+  rc = ki::enqueue_run(f, p, sweep0, n, cnt);
+  if (!rc && rates) {
+    std::vector<unsigned long long> h(ncnt);
+    hipError_t e = hipMemcpyAsync(h.data(), cnt.base, sizeof(unsigned long long) * ncnt, hipMemcpyDeviceToHost,
                                   ki::stream());
     if (e == hipSuccess) e = hipStreamSynchronize(ki::stream());
     if (e != hipSuccess) rc = ki::hip_fail(e, "acceptance counters");
-    for (int i = 0; i < n && !rc; ++i) acc_rates[i] = acceptance(f, p->nhits, h[i]);
+    for (int i = 0; i < n && !rc; ++i) {
+      unsigned long long t = 0;
+      for (int r = 0; r < ki::kCounterRows; ++r) t += h[(long long)r * cnt.row + i];
+      acc_rates[i] = acceptance(f, p->nhits, t);
+    }
   }
   if (rc) return rc;
   return ki::sync_stream();
@@ -245,7 +285,7 @@ extern "C" int klft_metropolis_schedule(klft_field_t f, int32_t *visit) {
   // nhits = 0: the real pass kernels run their thread-to-site map and record
   // the pass index without changing any link
   klft_metropolis_params p{0, 1.0, 0.1, 0};
-  rc = ki::enqueue_sweep(f, &p, 0, 0, f->counter, dv);
+  rc = ki::enqueue_sweep(f, &p, 0, 0, ki::Counters{f->counter, 0, ki::kCounterCols}, dv);
   if (!rc) {
     hipError_t e = hipMemcpyAsync(visit, dv, sizeof(int) * f->g.V, hipMemcpyDeviceToHost, ki::stream());
     if (e == hipSuccess) e = hipStreamSynchronize(ki::stream());

@@ -1,11 +1,10 @@
 // Metropolis sweep kernels for F64 links.
-#include "metro_kernels.hpp"
+#include "metro_launch.hpp"
 
 namespace klft_internal {
 int launch_passes_f64(klft_field_t f, void *links, int variant, int p0, int p1, const klft_metropolis_params *p,
-                      uint64_t sweep, int nsweeps, uint32_t chain, unsigned long long *counter,
-                      int counter_stride, int *visit) {
+                      uint64_t sweep, int nsweeps, uint32_t chain, klft_internal::Counters counter, int *visit) {
   return klft_metro::launch_passes_typed<double, false>(f, links, variant, p0, p1, p, sweep, nsweeps, chain, counter,
-                                                     counter_stride, visit);
+                                                     visit);
 }
 }  // namespace klft_internal
