@@ -19,6 +19,9 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <type_traits>
+#include <utility>
+
 #include "philox.hpp"
 
 namespace kd {
@@ -222,6 +225,19 @@ __device__ __forceinline__ void acc_mul_ad(Mat<R, N>& t, const Mat<R, N>& a, con
       cx<R> v = t.m[i][j];
 #pragma unroll
       for (int k = 0; k < N; ++k) v = cfma_c(a.m[i][k], b.m[j][k], v);
+      t.m[i][j] = v;
+    }
+}
+// t += a^dagger * b^dagger
+template <typename R, int N>
+__device__ __forceinline__ void acc_mul_dd(Mat<R, N>& t, const Mat<R, N>& a, const Mat<R, N>& b) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      cx<R> v = t.m[i][j];
+#pragma unroll
+      for (int k = 0; k < N; ++k) v = cfma_cc(a.m[k][i], b.m[j][k], v);
       t.m[i][j] = v;
     }
 }
@@ -644,6 +660,26 @@ struct Links {
       for (int c = 0; c < NCOMP; ++c) q[c * 64 + l] = u.m[c / NC][c % NC];
     }
   }
+  // the same past the caches: for a field that this kernel does not read
+  __device__ __forceinline__ void store_stream(long long s, int mu, const Mat<R, NC>& u) const {
+    typedef R vec2 __attribute__((ext_vector_type(2)));
+    typedef R vec4 __attribute__((ext_vector_type(4)));
+    cx<R>* q = p + run(s, mu);
+    const int l = (int)(s & 63);
+    auto at = [&](int c) { return u.m[c / NC][c % NC]; };
+    if constexpr (PAIRED) {
+#pragma unroll
+      for (int k = 0; k < NPAIR; ++k) {
+        const vec4 v = {at(2 * k).re, at(2 * k).im, at(2 * k + 1).re, at(2 * k + 1).im};
+        __builtin_nontemporal_store(v, reinterpret_cast<vec4*>(q + k * 128) + l);
+      }
+    }
+#pragma unroll
+    for (int c = 2 * NPAIR; c < NCOMP; ++c) {
+      const vec2 v = {at(c).re, at(c).im};
+      __builtin_nontemporal_store(v, reinterpret_cast<vec2*>(q + c * 64 + l));
+    }
+  }
 };
 
 // number of link-array elements (complex) for V sites
@@ -751,6 +787,110 @@ __device__ __forceinline__ Mat<R, NC> staple_lowreg(const Links<R, NC, COMP>& f,
     acc_mul(t, ab, f.load(s_xmnu, nu));
   }
   return t;
+}
+
+// The staples of the directions D .. D + K - 1 of a site by one thread: with all
+// four 44 link loads per site (the own links included), with two at a time 60,
+// instead of 76 by a thread per link, because a lower term's U_nu(x-nu) serves
+// every direction and the first product of an upper term,
+// A = U_nu(x+mu) U_mu(x+nu)^+, is direction nu's too, as A^+.
+//
+// The compiler would issue every load first and multiply last, far beyond the
+// registers: `settle` makes it finish a matrix before the loads that follow.
+template <typename R, int N>
+__device__ __forceinline__ void settle(Mat<R, N>& a) {
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+#ifdef __HIP_DEVICE_COMPILE__
+      asm volatile("" : "+v"(a.m[i][j].re), "+v"(a.m[i][j].im)::"memory");
+#endif
+    }
+}
+// f(0), f(1), ... f(N-1) with compile-time arguments (the loop unroller gives up
+// on bodies of this size, and an index left dynamic puts arrays in scratch)
+template <class F, int... I>
+__device__ __forceinline__ void unrolled(F&& f, std::integer_sequence<int, I...>) {
+  (f(std::integral_constant<int, I>{}), ...);
+}
+// the terms in order: kind 0 the lower term of (mu, nu); 1 the upper term of mu
+// with a direction nu outside D .. D + K - 1; 2 the plane mu < nu of two of them
+template <int ND, int D, int K>
+struct StapleTerms {
+  int n = 0, kind[24] = {}, mu[24] = {}, nu[24] = {};
+  bool first[24] = {};  // the term begins a new nu (kinds 0, 1) or the planes
+  constexpr void add(int k, int m, int v) {
+    kind[n] = k;
+    mu[n] = m;
+    nu[n] = v;
+    first[n] = n == 0 || kind[n - 1] != k || (k != 2 && nu[n - 1] != v);
+    ++n;
+  }
+  constexpr StapleTerms() {
+    for (int v = 0; v < ND; ++v)
+      for (int m = D; m < D + K; ++m)
+        if (m != v) add(0, m, v);
+    for (int v = 0; v < ND; ++v)
+      if (v < D || v >= D + K)
+        for (int m = D; m < D + K; ++m) add(1, m, v);
+    for (int m = D; m < D + K; ++m)
+      for (int v = m + 1; v < D + K; ++v) add(2, m, v);
+  }
+};
+// U and S: the K own links and staples.
+// AHEAD: the next term's links are in flight while a term is multiplied.
+template <typename R, int NC, bool COMP, int ND, int D, int K, bool AHEAD>
+__device__ __forceinline__ void staples_of(const Links<R, NC, COMP>& f, const Nbr<ND>& n, Mat<R, NC>* U,
+                                           Mat<R, NC>* S) {
+  constexpr StapleTerms<ND, D, K> T;
+  constexpr int NB = AHEAD ? 2 : 1;
+  Mat<R, NC> a[NB], b[NB], c[2], o[ND];
+  // the links of term t: its first product's two and, where a new one begins,
+  // U_nu(x-nu) (lower terms) or the own links
+  auto load = [&](auto tc) {
+    constexpr int t = decltype(tc)::value, mu = T.mu[t], nu = T.nu[t], q = t % NB;
+    if constexpr (T.kind[t] == 0) {
+      if constexpr (T.first[t]) c[nu & 1] = f.load(n.s + n.dm[nu], nu);
+      a[q] = f.load(n.s + n.dm[nu] + n.dp[mu], nu);
+      b[q] = f.load(n.s + n.dm[nu], mu);
+    } else {
+      a[q] = f.load(n.s + n.dp[mu], nu);
+      b[q] = f.load(n.s + n.dp[nu], mu);
+      if constexpr (T.kind[t] == 1 && T.first[t]) o[nu] = f.load(n.s, nu);
+      if constexpr (T.kind[t] == 2 && T.first[t]) {
+#pragma unroll
+        for (int m = D; m < D + K; ++m) U[m - D] = o[m] = f.load(n.s, m);
+      }
+    }
+  };
+#pragma unroll
+  for (int k = 0; k < K; ++k) S[k] = zero<R, NC>();
+  if constexpr (AHEAD) load(std::integral_constant<int, 0>{});
+  unrolled(
+      [&](auto tc) {
+        constexpr int t = decltype(tc)::value, mu = T.mu[t], nu = T.nu[t], q = t % NB;
+        if constexpr (!AHEAD)
+          load(tc);
+        else if constexpr (t + 1 < T.n)
+          load(std::integral_constant<int, t + 1>{});
+        Mat<R, NC> ab;
+        if constexpr (T.kind[t] == 0)
+          ab = mul_dd(a[q], b[q]);
+        else
+          ab = mul_ad(a[q], b[q]);
+        if constexpr (T.kind[t] == 0) {
+          acc_mul(S[mu - D], ab, c[nu & 1]);
+        } else {
+          acc_mul_ad(S[mu - D], ab, o[nu]);
+          if constexpr (T.kind[t] == 2) {
+            acc_mul_dd(S[nu - D], ab, o[mu]);
+            settle(S[nu - D]);
+          }
+        }
+        settle(S[mu - D]);
+      },
+      std::make_integer_sequence<int, T.n>{});
 }
 
 // plaquette at one site (GaugePlaquette.hpp:52-85), real part only:

@@ -112,14 +112,30 @@ __global__ __launch_bounds__(256) void k_force(Links<R, NC, COMP> f, R *P, Geom 
   if (partials) block_partial<256>(k, lds, partials);
 }
 
+// loads and stores past the caches (NT), for arrays that a launch touches once
+template <bool NT, typename R>
+__device__ __forceinline__ R load_stream(const R *p) {
+  if constexpr (NT) return __builtin_nontemporal_load(p);
+  return *p;
+}
+template <bool NT, typename R>
+__device__ __forceinline__ void store_stream(R *p, R v) {
+  if constexpr (NT)
+    __builtin_nontemporal_store(v, p);
+  else
+    *p = v;
+}
+
 // One leapfrog step with the momentum and link updates fused and the links
 // double-buffered: F from the links in src, P <- P - dtp F, and
 // dst(x,mu) = exp(i dtu P(x,mu)) src(x,mu) (FP32 links reunitarised).  The
 // staples read src only, so no link is written while another thread may
 // still read it; the arithmetic is that of k_force followed by
 // k_update_gauge, so the result is the same.  One thread per link as in
-// k_force: a block holds one 64-site chunk, wave w taking direction w.
-template <typename R, int NC, bool COMP, int ND, bool LOWREG>
+// k_force: a block holds one 64-site chunk, wave w taking direction w.  For the
+// SU(3) lattices in two and three dimensions that leave most CUs without a wave
+// (links_per_thread); the others take k_step_dirs.
+template <typename R, int NC, bool COMP, int ND, bool NT>
 __global__ __launch_bounds__(256) void k_md_step(Links<R, NC, COMP> src, Links<R, NC, COMP> dst, R *P, Geom g,
                                                   R coef, R dtp, R dtu) {
   src.nd = ND;
@@ -129,26 +145,107 @@ __global__ __launch_bounds__(256) void k_md_step(Links<R, NC, COMP> src, Links<R
   int x[ND], mu;
   long long s;
   if (!link_site<ND>(g, lb, x, &s, &mu)) return;
-  const Nbr<ND> nb = make_nbr<ND>(g, x, s);
-  Mat<R, NC> S;
-  if constexpr (LOWREG)
-    S = staple_lowreg<R, NC, COMP, ND>(src, nb, mu);
-  else
-    S = staple<R, NC, COMP, ND>(src, nb, mu);
+  R pm[NG];
+#pragma unroll
+  for (int a = 0; a < NG; ++a) pm[a] = load_stream<NT>(P + ((long long)mu * NG + a) * g.V + s);
+  const Mat<R, NC> S = staple<R, NC, COMP, ND>(src, make_nbr<ND>(g, x, s), mu);
   const Mat<R, NC> U = src.load(s, mu);
   R v[NG];
   project(mul(U, S), coef, v);
 #pragma unroll
   for (int a = 0; a < NG; ++a) {
-    R *q = P + ((long long)mu * NG + a) * g.V + s;
-    const R pn = *q - dtp * v[a];
-    *q = pn;
+    const R pn = pm[a] - dtp * v[a];
+    store_stream<NT>(P + ((long long)mu * NG + a) * g.V + s, pn);
     v[a] = dtu * pn;
   }
   const Mat<R, NC> e = exp_iq(v, (Mat<R, NC> *)nullptr);
   Mat<R, NC> u = mul(e, U);
   if constexpr (sizeof(R) == 4) reunitarize(u);
-  dst.store(s, mu, u);
+  if constexpr (NT)
+    dst.store_stream(s, mu, u);
+  else
+    dst.store(s, mu, u);
+}
+
+// The step (GAUGE) and the force (P only; Fout and kin as in k_force) with K
+// directions per thread: a block holds 64 sites, wave h taking the directions
+// h K .. h K + K - 1.  Bound by the L1: a CU keeps about 60 requests of 128
+// bytes in flight, and nearly each one waits for the memory-side cache or HBM, so
+// the time goes with the number of link loads, 19 a link with a thread per
+// link, 15 with two directions per thread, 11 with four (staples_of).
+// SU(3) 28x24x20x32 FP32 170 -> 145 us per step, 32^4 FP32 454 -> 345,
+// FP64 (two directions: four need 488 registers, one wave per SIMD) 860 -> 746,
+// SU(2) 16^4 FP64 32 -> 17.
+// With ND directions the next term's links are in flight while a term is
+// multiplied; with two, twice the waves do the same and the registers
+// that takes would cost one (SU(3) FP64 32^4 950 us).
+constexpr int step_waves(int rbytes, int nc, int k) { return rbytes == 8 && nc == 3 && k > 2 ? 1 : 2; }
+template <typename R, int NC, bool COMP, int ND, int K, bool NT, bool GAUGE>
+__global__ __launch_bounds__(64 * ND / K, step_waves(sizeof(R), NC, K)) void k_step_dirs(
+    Links<R, NC, COMP> src, Links<R, NC, COMP> dst, R *P, Geom g, R coef, R dtp, R dtu, double *Fout,
+    double *partials) {
+  src.nd = ND;
+  dst.nd = ND;
+  constexpr int NG = Ngen<NC>::value, NSUB = 1 << ND, NW = ND / K;
+  const unsigned int lb = xcd_block(blockIdx.x, gridDim.x);
+  const int sub = (int)(lb % NSUB), h = NW == 1 ? 0 : __builtin_amdgcn_readfirstlane((int)(threadIdx.x >> 6));
+  const long long r = (long long)(lb / NSUB) * 64 + (threadIdx.x & 63);
+  double kin = 0.0;
+  if (r < g.Vh) {
+    int x[ND];
+    sub_coords<ND>(g, sub, r, x);
+    const long long s = (long long)sub * g.Vh + r;
+    R pm[2][NG];
+    auto load_p = [&](int k, R *o) {
+#pragma unroll
+      for (int a = 0; a < NG; ++a) o[a] = load_stream<NT>(P + ((long long)(h * K + k) * NG + a) * g.V + s);
+    };
+    Mat<R, NC> U[K], S[K];
+    const Nbr<ND> nb = make_nbr<ND>(g, x, s);
+    if (NW == 1 || h == 0)
+      staples_of<R, NC, COMP, ND, 0, K, K == ND>(src, nb, U, S);
+    else
+      staples_of<R, NC, COMP, ND, ND - K, K, K == ND>(src, nb, U, S);
+    // the next direction's momenta are in flight while this one is updated
+    load_p(0, pm[0]);
+#pragma unroll
+    for (int k = 0; k < K; ++k) {
+      if (k + 1 < K) load_p(k + 1, pm[(k + 1) & 1]);
+      const int mu = h * K + k;
+      R v[NG];
+      project(mul(U[k], S[k]), coef, v);
+      if constexpr (!GAUGE) {
+        if (Fout) {
+          const long long site = lex_index<ND>(g, x);
+#pragma unroll
+          for (int a = 0; a < NG; ++a) Fout[(site * ND + mu) * NG + a] = (double)v[a];
+          continue;
+        }
+      }
+      double n2 = 0.0;
+#pragma unroll
+      for (int a = 0; a < NG; ++a) {
+        const R pn = pm[k & 1][a] - dtp * v[a];
+        store_stream<NT>(P + ((long long)mu * NG + a) * g.V + s, pn);
+        if constexpr (!GAUGE) n2 += (double)pn * (double)pn;
+        v[a] = dtu * pn;
+      }
+      kin += 0.5 * n2;
+      if constexpr (GAUGE) {
+        Mat<R, NC> u = mul(exp_iq(v, (Mat<R, NC> *)nullptr), U[k]);
+        if constexpr (sizeof(R) == 4) reunitarize(u);
+        if constexpr (NT)
+          dst.store_stream(s, mu, u);
+        else
+          dst.store(s, mu, u);
+      }
+      asm volatile("" ::: "memory");
+    }
+  }
+  if constexpr (!GAUGE) {
+    __shared__ double lds[NW];
+    if (partials) block_partial<64 * NW>(kin, lds, partials);
+  }
 }
 
 // U <- exp(i dtau P) U; FP32 links are reunitarised after the update
@@ -235,14 +332,45 @@ int enqueue_refresh(klft_hmc_t h, uint64_t traj, int slot) {
   });
 }
 
+// Directions per thread of k_step_dirs (1: a thread per link, k_md_step and
+// k_force).
+// Four dimensions: FP64 SU(3) takes two (746 against 787 us with one and 1300
+// with four at 32^4; 26.6, 33.6 and 59.7 at 12^4).  The others take all four once
+// the waves of two would wait for one another: U(1) and SU(2) from a wave per
+// SIMD on (SU(2) FP64 16^4 17.3 against 18.4 us, 12^4 14.1 against 13.8, 8^4 10.6
+// against 9.0; U(1) 32^4 54 against 65), FP32 SU(3), with two waves per SIMD at
+// most, where the fields no longer fit the memory-side cache (32^4 345 against
+// 372, 28x24x20x32 145 both, 20^4 60 against 53, 12^4 23.6 against 19.5).
+// Fewer dimensions: all of them, but for SU(3) with less than a wave per CU, where
+// a step lasts as long as one thread (16^3 FP64 19.1 against 14.3 us with one
+// direction, 64^2 8.7 against 6.9; 32^3 23.1 against 28.7).
+int directions_per_thread(const klft_field_s *f, bool streams) {
+  if (f->nd < 4) return f->nc == 3 && f->g.V < 64 * 256 ? 1 : f->nd;
+  if (f->nc == 3) return f->storage == KLFT_STORAGE_F64 || !streams ? 2 : 4;
+  return f->g.V < 64 * 1024 ? 2 : 4;
+}
+
+// Links read, links written (`links` buffers in all) and momenta beyond 300 MiB
+// (the memory-side cache holds 256 MB): what a launch touches once goes past
+// the caches (SU(3) 32^4 FP64 776 -> 746 us per step, FP32 363 -> 345, SU(2) FP32,
+// 304 MiB, 137 -> 129); below that the next launch finds it there (SU(3)
+// 28x24x20x32 FP32, 289 MiB, 145 both, 16^4 FP64 46 against 50, U(1) 32^4 54
+// against 70).  KLFT_VARIANT="md_stream=0|1" forces one.
+bool past_caches(const klft_field_s *f, int links) {
+  const int forced = ki::forced_variant("md_stream");
+  if (forced >= 0) return forced != 0;
+  const size_t rbytes = f->storage == KLFT_STORAGE_F64 ? 8 : 4;
+  return links * f->link_bytes + (size_t)f->g.V * f->nd * ngen(f->nc) * rbytes > (size_t)300 << 20;
+}
+
 // variants: 0 one thread per link, one-term-at-a-time staple; 4 the same with
-// all staple loads in flight at once (full staple).  1-3 (occupancy targets,
-// one thread per site) never won and were removed.
-constexpr int kForceVariants = 5;
+// all staple loads in flight at once (full staple); 5 a thread for all
+// directions of a site; 6 for two (four dimensions)
+constexpr int kForceVariants = 7;
 
 int launch_force(klft_hmc_t h, double dtau, double *Fout, int kin_slot, int variant) {
   klft_field_t f = h->f;
-  if (variant != 0 && variant != 4) return ki::set_error(KLFT_E_ARG, "force variant %d is not built", variant);
+  if (variant != 0 && variant < 4) return ki::set_error(KLFT_E_ARG, "force variant %d is not built", variant);
   // with a kinetic slot, every block writes a partial; k_sum_blocks adds them
   double *parts = kin_slot >= 0 ? f->partials : nullptr;
   return ki::dispatch(f->storage, f->nc, f->nd, [&](auto rt, auto nct, auto ct, auto ndt) -> int {
@@ -253,12 +381,28 @@ int launch_force(klft_hmc_t h, double dtau, double *Fout, int kin_slot, int vari
     if (nb > f->max_partials) return ki::set_error(KLFT_E_ARG, "lattice too large for reduction");
     {
       ki::ProfScope prof("force", "derivative+update_momentum");
-      if (variant == 4)
-        hipLaunchKernelGGL((k_force<R, NC, COMP, ND, false>), dim3((unsigned)nb), dim3(64 * ND), 0, ki::stream(),
-                           links, (R *)h->P, f->g, coef, (R)dtau, Fout, parts);
+      auto dirs = [&](auto kt, auto ntt) {
+        constexpr int K = decltype(kt)::value;
+        hipLaunchKernelGGL((k_step_dirs<R, NC, COMP, ND, K, decltype(ntt)::value != 0, false>), dim3((unsigned)nb),
+                           dim3(64 * ND / K), 0, ki::stream(), links, links, (R *)h->P, f->g, coef, (R)dtau, R(0), Fout,
+                           parts);
+      };
+      auto go = [&](auto ntt) {
+        if (variant == 5)
+          dirs(ki::ic<ND>{}, ntt);
+        else if (variant == 6)
+          dirs(ki::ic<ND == 4 ? 2 : ND>{}, ntt);
+        else if (variant == 4)
+          hipLaunchKernelGGL((k_force<R, NC, COMP, ND, false>), dim3((unsigned)nb), dim3(64 * ND), 0, ki::stream(),
+                             links, (R *)h->P, f->g, coef, (R)dtau, Fout, parts);
+        else
+          hipLaunchKernelGGL((k_force<R, NC, COMP, ND, true>), dim3((unsigned)nb), dim3(64 * ND), 0, ki::stream(),
+                             links, (R *)h->P, f->g, coef, (R)dtau, Fout, parts);
+      };
+      if (past_caches(f, 1))
+        go(ki::ic<1>{});
       else
-        hipLaunchKernelGGL((k_force<R, NC, COMP, ND, true>), dim3((unsigned)nb), dim3(64 * ND), 0, ki::stream(),
-                           links, (R *)h->P, f->g, coef, (R)dtau, Fout, parts);
+        go(ki::ic<0>{});
       KLFT_HIP(hipGetLastError());
     }
     if (parts) return ki::enqueue_sum_blocks(parts, nb, f->result + kin_slot);
@@ -268,8 +412,7 @@ int launch_force(klft_hmc_t h, double dtau, double *Fout, int kin_slot, int vari
 
 // the tuning launcher uses dtau = 0, which leaves the momenta unchanged
 int enqueue_force(klft_hmc_t h, double dtau, double *Fout, int kin_slot) {
-  // untuned default, the fastest at 32^4: the full staple for FP64 links
-  const int dflt = h->f->storage == KLFT_STORAGE_F64 ? 4 : 0;
+  const int k = directions_per_thread(h->f, past_caches(h->f, 1)), dflt = k == 1 ? 4 : (k == 2 && h->f->nd == 4 ? 6 : 5);
   const int v = ki::pick_variant("force", h->f, kForceVariants, dflt,
                                  [&](int var) { return launch_force(h, 0.0, nullptr, -1, var); });
   return launch_force(h, dtau, Fout, kin_slot, v);
@@ -303,8 +446,10 @@ int enqueue_kinetic(klft_hmc_t h, int slot) {
   });
 }
 
-// variants: 0 one-term-at-a-time staple, 1 full staple (all loads in flight)
-constexpr int kMdVariants = 2;
+// variants: 1 a thread per link, 2 a thread for all directions of a site, 3 for
+// two directions (four dimensions).  0 (a thread per link with one term of
+// the staple at a time) never won and runs as 1.
+constexpr int kMdVariants = 4;
 
 int launch_md_step(klft_hmc_t h, void *src, void *dst, double dtp, double dtu, int variant) {
   klft_field_t f = h->f;
@@ -316,12 +461,25 @@ int launch_md_step(klft_hmc_t h, void *src, void *dst, double dtp, double dtu, i
     const unsigned nb = (unsigned)link_blocks<ND>(f->g);
     const R coef = (R)(h->p.beta / (double)NC);
     ki::ProfScope prof("md_step", "derivative+update_momentum+update_gauge");
-    if (variant == 1)
-      hipLaunchKernelGGL((k_md_step<R, NC, COMP, ND, false>), dim3(nb), dim3(64 * ND), 0, ki::stream(), ls, ld,
-                         (R *)h->P, f->g, coef, (R)dtp, (R)dtu);
+    auto dirs = [&](auto kt, auto ntt) {
+      constexpr int K = decltype(kt)::value;
+      hipLaunchKernelGGL((k_step_dirs<R, NC, COMP, ND, K, decltype(ntt)::value != 0, true>), dim3(nb),
+                         dim3(64 * ND / K), 0, ki::stream(), ls, ld, (R *)h->P, f->g, coef, (R)dtp, (R)dtu, nullptr,
+                         nullptr);
+    };
+    auto go = [&](auto ntt) {
+      if (variant == 2)
+        dirs(ki::ic<ND>{}, ntt);
+      else if (variant == 3)
+        dirs(ki::ic<ND == 4 ? 2 : ND>{}, ntt);
+      else
+        hipLaunchKernelGGL((k_md_step<R, NC, COMP, ND, decltype(ntt)::value != 0>), dim3(nb), dim3(64 * ND), 0,
+                           ki::stream(), ls, ld, (R *)h->P, f->g, coef, (R)dtp, (R)dtu);
+    };
+    if (past_caches(f, 2))
+      go(ki::ic<1>{});
     else
-      hipLaunchKernelGGL((k_md_step<R, NC, COMP, ND, true>), dim3(nb), dim3(64 * ND), 0, ki::stream(), ls, ld,
-                         (R *)h->P, f->g, coef, (R)dtp, (R)dtu);
+      go(ki::ic<0>{});
     KLFT_HIP(hipGetLastError());
     return KLFT_OK;
   });
@@ -336,8 +494,8 @@ int launch_md_step(klft_hmc_t h, void *src, void *dst, double dtp, double dtu, i
 int enqueue_leapfrog(klft_hmc_t h, int kin_slot, int *start_slot) {
   const double dtau = h->p.tau / (double)h->p.nsteps;
   klft_field_t f = h->f;
-  // untuned default: the staple form of the force kernel's default
-  const int v = ki::pick_variant("md_step", f, kMdVariants, f->storage == KLFT_STORAGE_F64 ? 1 : 0, [&](int var) {
+  const int k = directions_per_thread(f, past_caches(f, 2)), dflt = k == 1 ? 1 : (k == 2 && f->nd == 4 ? 3 : 2);
+  const int v = ki::pick_variant("md_step", f, kMdVariants, dflt, [&](int var) {
     return launch_md_step(h, f->links, h->Ubuf[0], 0.0, 0.0, var);  // dtp = 0: P unchanged
   });
   void *cur = f->links;
