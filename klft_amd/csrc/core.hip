@@ -864,47 +864,69 @@ extern "C" int klft_staple_field(klft_field_t f, klft_field_t out) {
 // ============================================================================
 // One block holds C full columns along nu (periodic), one thread per site.
 // For each requested L (ascending) a thread extends its mu-line
-// F_L(x) = U_mu(x) ... U_mu(x+(L-1)mu) and publishes it in LDS; then for
-// T = 0, 1, ... it carries the three-sided staple
+// F_L(x) = U_mu(x) ... U_mu(x+(L-1)mu); then for T = 0, 1, ... the three-sided
+// staple
 //   D(L,T) = l_nu(x;T)^+ F_L(x) l_nu(x+L mu;T),
 //   D(L,T) = U_nu(x+(T-1)nu)^+ D(L,T-1) U_nu(x+L mu+(T-1)nu),
-// and closes the loop with the top line read from LDS:
+// moves up the column, one thread a step, and is closed with the top line:
 //   w(x;L,T) = Re Tr[D(L,T) F_L(x+T nu)^+],
 // which equals the reference's Re Tr[A B^+] with A = l_mu(x;L) l_nu(x+L mu;T),
-// B = l_nu(x;T) l_mu(x+T nu;L) (WilsonLoop.hpp:129-160).  No line field is
-// materialised in HBM.  Wave partial sums go to
+// B = l_nu(x;T) l_mu(x+T nu;L) (WilsonLoop.hpp:129-160).  The thread at y
+// holds the links U_nu(y-nu), U_nu(y-nu+L mu) and the line F_L(y), so that D
+// alone moves, and with every step D comes from the site below.  No line
+// field is materialised in HBM.  Wave partial sums go to
 // partials[(((plane * nL + li) * (Tmax+1) + T) * gridDim.x + blockIdx.x)
 //          * waves per block + wave].
-template <typename R, int NC, bool COMP, int ND, bool LNU = true>
-__global__ __launch_bounds__(512) void k_wilson(Links<R, NC, COMP> f, Geom g, int mu0, int nu,
+//
+// kWave: D moves between lanes, and a wave holds whole columns; else through LDS, in
+// two buffers (kLds2, a barrier a step) or one where two do not fit (kLds1).
+//
+// Bound by the vector unit, 216 FMAs for D and 36 for the trace of SU(3), with the
+// lane moves and 30 instructions of the wave's sum beside them: 64 loops of three
+// planes at 32^4 FP64 2.50 ms, their FP64 instructions alone 1.8 (FP32 1.28 ms).
+// With the thread at x loading U_nu(x+L mu+(T-1) nu) at each step, the
+// nu-links and lines in LDS, every step waited for the L2: 3.58 ms (FP32 1.77; U(1)
+// 0.57 -> 0.25, SU(2) 1.52 -> 0.85; SU(3) 16^4 FP64 0.25 -> 0.16, U(1) 8^4 0.044 ->
+// 0.023).  More waves do not help: three per SIMD spill (2.83 ms).
+enum class Move { kWave, kLds2, kLds1 };
+template <typename R, int NC, bool COMP, int ND, Move MOVE>
+__global__ __launch_bounds__(MOVE == Move::kWave ? 64 : 512, 2) void k_wilson(Links<R, NC, COMP> f, Geom g, int mu0, int nu,
                                                  int ncolblk, int nL, const int *__restrict__ Ls,
                                                  int Tmax, double *partials, double *per_site,
                                                  int ps_li, int ps_T) {
   f.nd = ND;
   extern __shared__ __align__(16) unsigned char smem[];
-  // lds: the threads' current mu-lines; lnu (LNU): the columns' nu-links
-  // U_nu(x), read by every step T of the staple recurrence (else loaded)
   Mat<R, NC> *lds = reinterpret_cast<Mat<R, NC> *>(smem);
-  Mat<R, NC> *lnu = lds + blockDim.x;
   const int plane = blockIdx.y;
   const int mu = mu0 < 0 ? plane : mu0;
   const int Ln = g.L[nu];
   const int tid = threadIdx.x;
   const int cl = tid / Ln, k = tid - cl * Ln;
   const long long ncol = g.V / Ln;
-  const long long col = (long long)blockIdx.x * ncolblk + cl;
+  const unsigned int bx = xcd_block(blockIdx.x, gridDim.x);
+  const long long col = (long long)bx * ncolblk + cl;
   const bool valid = cl < ncolblk && col < ncol;
   int x[ND];
   {
     uint32_t r = valid ? (uint32_t)col : 0u;
+    // along the last dimension a column is contiguous: columns that follow one
+    // another along mu then read one another's links while they are in the L2
+    // (SU(3) 32^4 FP64 2.85 -> 2.52 ms)
+    const int first = nu == ND - 1 ? mu : nu;
+    if (first != nu) {
+      x[first] = (int)(r % (uint32_t)g.L[first]);
+      r /= (uint32_t)g.L[first];
+    }
 #pragma unroll
     for (int d = ND - 1; d >= 0; --d) {
-      if (d == nu) continue;
+      if (d == nu || d == first) continue;
       x[d] = (int)(r % (uint32_t)g.L[d]);
       r /= (uint32_t)g.L[d];
     }
-    x[nu] = k;
+    x[nu] = valid ? k : 0;
   }
+  // the thread below in the column (threads without a column: their own)
+  const int below = !valid ? tid : (k == 0 ? tid + Ln - 1 : tid - 1);
   // A device index is a sum over dimensions of the coordinate's sublattice
   // bit (times Vh) and its encoded half-coordinate, so the shifted sites'
   // indices below replace only the shifted coordinates' terms of x's.
@@ -917,49 +939,43 @@ __global__ __launch_bounds__(512) void k_wilson(Links<R, NC, COMP> f, Geom g, in
 #pragma unroll
   for (int d = 0; d < ND; ++d) base += dterm(d, x[d]);
   const long long base_nomu = base - dterm(mu, x[mu]);  // x without its mu term
-  const long long term_nu = dterm(nu, x[nu]);
-  if constexpr (LNU) {
-    if (valid) lnu[tid] = f.load(base, nu);
-  }
+  const long long down = dterm(nu, x[nu] == 0 ? Ln - 1 : x[nu] - 1) - dterm(nu, x[nu]);
+  const Mat<R, NC> a = f.load(base + down, nu);  // U_nu(y - nu)
   Mat<R, NC> F = identity<R, NC>();
-  int Lcur = 0;
+  int Lcur = 0, buf = 0;
   for (int li = 0; li < nL; ++li) {
     const int L = Ls[li];
-    if (valid) {
-      while (Lcur < L) {
-        F = mul(F, f.load(base_nomu + dterm(mu, wrap(x[mu] + Lcur, Lmu)), mu));  // U_mu(x + Lcur mu)
-        ++Lcur;
-      }
+    const Mat<R, NC> b = f.load(base_nomu + dterm(mu, wrap(x[mu] + L, Lmu)) + down, nu);  // U_nu(y - nu + L mu)
+    while (Lcur < L) {
+      F = mul(F, f.load(base_nomu + dterm(mu, wrap(x[mu] + Lcur, Lmu)), mu));  // U_mu(x + Lcur mu)
+      ++Lcur;
     }
-    __syncthreads();
-    lds[tid] = F;
-    __syncthreads();
     Mat<R, NC> D = F;
-    // index of x + L mu without its nu term
-    const long long base_L = base_nomu + dterm(mu, wrap(x[mu] + L, Lmu)) - term_nu;
     for (int T = 0; T <= Tmax; ++T) {
-      double w = 0.0;
-      if (valid) {
-        if (T > 0) {
-          const int kp = wrap(k + T - 1, Ln);
-          const long long tnu = dterm(nu, kp);
-          const Mat<R, NC> b = f.load(base_L + tnu, nu);   // U_nu(x + L mu + (T-1) nu)
-          Mat<R, NC> a;                                     // U_nu(x + (T-1) nu), same column
-          if constexpr (LNU)
-            a = lnu[cl * Ln + kp];
-          else
-            a = f.load(base - term_nu + tnu, nu);
-          D = mul(mul_da(a, D), b);
+      if (T > 0) {
+        if constexpr (MOVE == Move::kWave) {
+          D = lane_mat(D, below);
+        } else {
+          if constexpr (MOVE == Move::kLds2) buf ^= (int)blockDim.x;
+          lds[buf + tid] = D;
+          __syncthreads();
+          D = lds[buf + below];
+          if constexpr (MOVE == Move::kLds1) __syncthreads();
         }
-        const int kt = wrap(k + T, Ln);
-        w = (double)retr_mul_ad(D, lds[cl * Ln + kt]);
-        if (per_site && li == ps_li && T == ps_T && plane == 0) per_site[lex_index<ND>(g, x)] = w;
+        D = mul(mul_da(a, D), b);
+      }
+      const double w = valid ? (double)retr_mul_ad(D, F) : 0.0;
+      if (per_site && li == ps_li && T == ps_T && plane == 0 && valid) {
+        int y[ND];
+#pragma unroll
+        for (int d = 0; d < ND; ++d) y[d] = d == nu ? (k + Ln - T % Ln) % Ln : x[d];  // where the loop began
+        per_site[lex_index<ND>(g, y)] = w;
       }
       // one partial per wave (no block barrier per (L,T)); the partials of
       // an output are summed in a fixed order afterwards
-      const double ws = wave_sum(w);
-      if ((tid & 63) == 0)
-        partials[(((long long)(plane * nL + li) * (Tmax + 1) + T) * gridDim.x + blockIdx.x) * (blockDim.x >> 6) +
+      const double ws = wave_sum_last(w);
+      if ((tid & 63) == 63)
+        partials[(((long long)(plane * nL + li) * (Tmax + 1) + T) * gridDim.x + bx) * (blockDim.x >> 6) +
                  (tid >> 6)] = ws;
     }
   }
@@ -1011,19 +1027,28 @@ int wilson_sums(klft_field_t f, int mu0, int nplanes, int nu, const int *pairs, 
   const int nL = (int)Ls.size();
   const int Ln = f->dims[nu];
   const size_t mbytes = (size_t)f->nc * f->nc * f->cbytes;
+  // Columns that fill at least 7/8 of a wave's lanes move D between them: SU(3)
+  // FP64 16^4 157 against 188 us, FP32 16^3 x 28 (56 lanes) 168 against 181; others take
+  // a block's worth of columns and move it through LDS (16^3 x 24 and 48, 48
+  // lanes, FP32 160 against 167 and 413 against 462 us, 16^3 x 40 255 against 310).
+  // KLFT_VARIANT="wilson=0|1" asks for the lanes or for LDS.
   int C = std::max(1, 256 / Ln);
   // whole waves: the trailing threads (cl >= C) hold no column
   int block = ((C * Ln + 63) / 64) * 64;
-  // the block's mu-lines and nu-links in LDS, 2 * block matrices: fewer
-  // columns per block where that does not fit; a column too long for both
-  // keeps only the mu-lines (the nu-links are loaded at every step)
   while (C > 1 && 2 * block * mbytes > 64 * 1024) {
     C /= 2;
     block = ((C * Ln + 63) / 64) * 64;
   }
-  const bool lnu = 2 * block * mbytes <= 64 * 1024;
+  Move move = 2 * block * mbytes <= 64 * 1024 ? Move::kLds2 : Move::kLds1;
   if (block > 512 || block * mbytes > 64 * 1024)
     return ki::set_error(KLFT_E_ARG, "extent %d along nu too large for the Wilson-loop kernel", Ln);
+  const int fw = ki::forced_variant("wilson");
+  const int inwave = 64 / Ln;
+  if (fw < 0 ? inwave * Ln >= 56 : fw == 0 && inwave > 0) {
+    move = Move::kWave;
+    C = inwave;
+    block = 64;
+  }
   const long long ncol = f->g.V / Ln;
   const unsigned nbx = (unsigned)((ncol + C - 1) / C);
   const long long nout = (long long)nplanes * nL * (Tmax + 1);
@@ -1054,14 +1079,18 @@ int wilson_sums(klft_field_t f, int mu0, int nplanes, int nu, const int *pairs, 
   int rc = ki::dispatch(f->storage, f->nc, f->nd, [&](auto rt, auto nct, auto ct, auto ndt) -> int {
     KLFT_UNPACK(rt, nct, ct, ndt);
     ki::ProfScope prof("wilson", "WilsonLoop_GaugeField_WLoop_munu");
-    if (lnu)
-      hipLaunchKernelGGL((k_wilson<R, NC, COMP, ND, true>), dim3(nbx, nplanes), dim3(block),
-                         2 * block * sizeof(Mat<R, NC>), ki::stream(), ki::links_of<R, NC, COMP>(f), f->g,
+    auto go = [&](auto mt, int nbuf) {
+      constexpr Move M = decltype(mt)::value;
+      hipLaunchKernelGGL((k_wilson<R, NC, COMP, ND, M>), dim3(nbx, nplanes), dim3(block),
+                         nbuf * block * sizeof(Mat<R, NC>), ki::stream(), ki::links_of<R, NC, COMP>(f), f->g,
                          nplanes > 1 ? -1 : mu0, nu, C, nL, dLs, Tmax, dpart, dps, ps_li, ps_T);
+    };
+    if (move == Move::kWave)
+      go(std::integral_constant<Move, Move::kWave>{}, 0);
+    else if (move == Move::kLds2)
+      go(std::integral_constant<Move, Move::kLds2>{}, 2);
     else
-      hipLaunchKernelGGL((k_wilson<R, NC, COMP, ND, false>), dim3(nbx, nplanes), dim3(block),
-                         block * sizeof(Mat<R, NC>), ki::stream(), ki::links_of<R, NC, COMP>(f), f->g,
-                         nplanes > 1 ? -1 : mu0, nu, C, nL, dLs, Tmax, dpart, dps, ps_li, ps_T);
+      go(std::integral_constant<Move, Move::kLds1>{}, 1);
     KLFT_HIP(hipGetLastError());
     return KLFT_OK;
   });

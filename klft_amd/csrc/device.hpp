@@ -1368,6 +1368,37 @@ __device__ __forceinline__ double wave_sum(double v) {
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
   return v;
 }
+// the same in lane 63 alone, by lane moves of the vector unit instead of six
+// dependent trips through the LDS crossbar
+template <int CTRL, int ROWS>
+__device__ __forceinline__ double dpp_f64(double v) {
+  const long long b = __double_as_longlong(v);
+  const int lo = __builtin_amdgcn_update_dpp(0, (int)b, CTRL, ROWS, 0xf, false);
+  const int hi = __builtin_amdgcn_update_dpp(0, (int)(b >> 32), CTRL, ROWS, 0xf, false);
+  return __longlong_as_double(((long long)hi << 32) | (unsigned int)lo);
+}
+__device__ __forceinline__ double wave_sum_last(double v) {
+  v += dpp_f64<0xB1, 0xf>(v);   // lane ^ 1
+  v += dpp_f64<0x4E, 0xf>(v);   // lane ^ 2
+  v += dpp_f64<0x141, 0xf>(v);  // the other half of the eight
+  v += dpp_f64<0x140, 0xf>(v);  // the other half of the sixteen
+  v += dpp_f64<0x142, 0xa>(v);  // row 0 to 1, row 2 to 3
+  v += dpp_f64<0x143, 0xc>(v);  // row 1 to 2 and 3
+  return v;
+}
+// the matrix that lane `src` holds
+template <typename R, int N>
+__device__ __forceinline__ Mat<R, N> lane_mat(const Mat<R, N>& a, int src) {
+  Mat<R, N> r;
+#pragma unroll
+  for (int i = 0; i < N; ++i)
+#pragma unroll
+    for (int j = 0; j < N; ++j) {
+      r.m[i][j].re = __shfl(a.m[i][j].re, src, 64);
+      r.m[i][j].im = __shfl(a.m[i][j].im, src, 64);
+    }
+  return r;
+}
 __device__ __forceinline__ unsigned long long wave_sum_u64(unsigned long long v) {
 #pragma unroll
   for (int o = 32; o >= 1; o >>= 1) v += __shfl_xor(v, o, 64);
