@@ -200,6 +200,12 @@ extern "C" int klft_metropolis_run(klft_field_t f, const klft_metropolis_params 
   int rc = check_params(f, p);
   if (rc) return rc;
   if (n < 0) return ki::set_error(KLFT_E_ARG, "negative sweep count");
+  // longer runs with rates in slices, whose counters take 128 MiB
+  constexpr int kSlice = 1 << 20;
+  for (; acc_rates && n > kSlice; n -= kSlice, sweep0 += kSlice, acc_rates += kSlice) {
+    rc = klft_metropolis_run(f, p, sweep0, kSlice, acc_rates);
+    if (rc) return rc;
+  }
   // one column of counters per sweep, in a buffer kept with the field (grown
   // only when a longer run asks for more) and cleared by a kernel; rows of
   // whole lines
@@ -207,7 +213,6 @@ extern "C" int klft_metropolis_run(klft_field_t f, const klft_metropolis_params 
   ki::Counters cnt{f->counter, 0, ki::kCounterCols};
   long long ncnt = (long long)ki::kCounterRows * ki::kCounterCols;
   if (rates) {
-    if (n > (1 << 26)) return ki::set_error(KLFT_E_ARG, "at most 2^26 sweeps per run with rates");
     cnt.row = (n + 15) / 16 * 16;
     ncnt = (long long)ki::kCounterRows * cnt.row;
     if (ncnt > f->run_capacity) {
