@@ -22,6 +22,7 @@
 #include <type_traits>
 #include <utility>
 
+#include "metro_rules.hpp"
 #include "philox.hpp"
 
 namespace kd {
@@ -1136,10 +1137,9 @@ __device__ __forceinline__ bool rand_sun_w(const uint32_t* w, R delta, Mat<R, 3>
   return true;
 }
 
-// 1 / |v| of a row with |v|^2 = n2; false when the rejection loop would draw
-// the row again (1 + |v| rounds to 1)
+// 1 / |v| of a row with |v|^2 = n2; false when the row is drawn again
 __device__ __forceinline__ bool row_scale(double n2, double& f) {
-  if (!(n2 > 0x1p-106)) return false;  // |v| <= 2^-53
+  if (klft_metro::row_redrawn(n2)) return false;
   f = inv_sqrt(n2);
   return true;
 }
