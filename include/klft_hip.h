@@ -117,7 +117,10 @@ int klft_wilson_loop_temporal(klft_field_t f, const int *pairs, int npairs, int 
 typedef struct {
   int nhits;    /* MetropolisParams::nHits */
   double beta;  /* MetropolisParams::beta */
-  double delta; /* MetropolisParams::delta */
+  double delta; /* MetropolisParams::delta; SU(3) with the reference's law draws rows
+                   of uniforms of [0, delta) until one has a norm above 2^-53 (FP32
+                   links: 2^-24), so a delta of 0, or one too small or too large for
+                   that, is KLFT_E_ARG there */
   uint64_t seed;
 } klft_metropolis_params;
 

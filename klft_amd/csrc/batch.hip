@@ -313,6 +313,14 @@ int check_batch(klft_batch_t b) {
   return KLFT_OK;
 }
 
+// before hits are drawn: a delta whose SU(3) proposals the kernels could not draw
+int check_delta(klft_batch_t b, int nhits, double delta) {
+  if (nhits <= 0 || klft_metro::rows_kept(delta, b->storage == KLFT_STORAGE_F64)) return KLFT_OK;
+  for (klft_field_t f : b->fields)
+    if (f->nc == 3) return ki::set_error(KLFT_E_ARG, "delta=%g: no SU(3) proposal can be drawn", delta);
+  return KLFT_OK;
+}
+
 void drop_graphs(klft_batch_t b) {
   if (b->exec) (void)hipGraphExecDestroy(b->exec);
   if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -604,6 +612,8 @@ extern "C" int klft_batch_sweep(klft_batch_t b, int nhits, double delta, uint64_
   int rc = check_batch(b);
   if (rc) return rc;
   if (nhits < 0) return ki::set_error(KLFT_E_ARG, "nHits must be >= 0");
+  rc = check_delta(b, nhits, delta);
+  if (rc) return rc;
   const uint32_t s = (uint32_t)sweep;
   KLFT_HIP(hipMemcpyAsync(b->d_sweep, &s, sizeof s, hipMemcpyHostToDevice, ki::stream()));
   rc = enqueue_step(b, nhits, delta, seed);
@@ -621,6 +631,8 @@ extern "C" int klft_batch_run(klft_batch_t b, int nhits, double delta, uint64_t 
   int rc = check_batch(b);
   if (rc) return rc;
   if (nhits < 0 || n < 0) return ki::set_error(KLFT_E_ARG, "invalid sweep count");
+  if (n > 0) rc = check_delta(b, nhits, delta);
+  if (rc) return rc;
   rc = ensure_graph(b, nhits, delta, seed);
   if (rc) return rc;
   const uint32_t s = (uint32_t)sweep0;
@@ -731,6 +743,8 @@ extern "C" int klft_ptbc_step(klft_batch_t b, int nhits, double delta, uint64_t 
   int rc = check_batch(b);
   if (rc) return rc;
   if (!b->ptbc) return ki::set_error(KLFT_E_STATE, "not a PTBC replica set");
+  rc = check_delta(b, nhits, delta);
+  if (rc) return rc;
   rc = ensure_graph(b, nhits, delta, seed);
   if (rc) return rc;
   const uint32_t s = (uint32_t)step;

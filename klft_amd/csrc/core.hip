@@ -487,6 +487,10 @@ static int launch_init(klft_field_t f, int kind, double param, uint64_t seed, do
 
 extern "C" int klft_field_set_identity(klft_field_t f) { return launch_init(f, 0, 0.0, 0); }
 extern "C" int klft_field_set_random_sun(klft_field_t f, double delta, uint64_t seed) {
+  const int rc = ki::check_field(f);
+  if (rc) return rc;
+  if (f->nc == 3 && !klft_metro::rows_kept(delta, true))
+    return ki::set_error(KLFT_E_ARG, "delta=%g: no SU(3) link can be drawn", delta);
   return launch_init(f, 1, delta, seed);
 }
 extern "C" int klft_field_set_random_algebra(klft_field_t f, double eps, uint64_t seed) {

@@ -169,6 +169,14 @@ static int check_params(klft_field_t f, const klft_metropolis_params *p) {
   return KLFT_OK;
 }
 
+// before hits are drawn: a delta whose proposals the kernels could not draw
+static int check_delta(klft_field_t f, const klft_metropolis_params *p) {
+  if (f->nc == 3 && f->proposal == KLFT_PROPOSAL_REFERENCE && p->nhits > 0 &&
+      !klft_metro::rows_kept(p->delta, f->storage == KLFT_STORAGE_F64))
+    return ki::set_error(KLFT_E_ARG, "delta=%g: no SU(3) proposal can be drawn", p->delta);
+  return KLFT_OK;
+}
+
 static double acceptance(klft_field_t f, int nhits, unsigned long long n) {
   // Metropolis.hpp:169-175
   double norm = 1.0;
@@ -181,6 +189,7 @@ static double acceptance(klft_field_t f, int nhits, unsigned long long n) {
 extern "C" int klft_metropolis_sweep(klft_field_t f, const klft_metropolis_params *p, uint64_t sweep,
                                      double *acc_rate, int64_t *naccepted) {
   int rc = check_params(f, p);
+  if (!rc) rc = check_delta(f, p);
   if (rc) return rc;
   constexpr int nc = ki::kCounterRows * ki::kCounterCols;
   hipLaunchKernelGGL(k_zero_u64, dim3(1), dim3(nc), 0, ki::stream(), f->counter, nc);
@@ -200,6 +209,8 @@ extern "C" int klft_metropolis_run(klft_field_t f, const klft_metropolis_params 
   int rc = check_params(f, p);
   if (rc) return rc;
   if (n < 0) return ki::set_error(KLFT_E_ARG, "negative sweep count");
+  if (n > 0) rc = check_delta(f, p);
+  if (rc) return rc;
   // longer runs with rates in slices, whose counters take 128 MiB
   constexpr int kSlice = 1 << 20;
   for (; acc_rates && n > kSlice; n -= kSlice, sweep0 += kSlice, acc_rates += kSlice) {

@@ -30,5 +30,10 @@ int main(int argc, char **argv) {
     printf("%d %d\n", n, (int)again);
     return 0;
   }
+  if (!strcmp(argv[1], "rows_kept")) {  // fp64 delta ...
+    for (int i = 3; i < argc; ++i)
+      printf("%d\n", (int)klft_metro::rows_kept(strtod(argv[i], nullptr), atoi(argv[2]) != 0));
+    return 0;
+  }
   return 1;
 }

@@ -42,3 +42,41 @@ def test_nonfinite_delta_in_a_batch_is_rejected(monkeypatch, variant, storage, d
     r.step(3, delta, 7, 0)
     assert np.array_equal(r.download(0), before)
     r.close()
+
+
+def test_delta_without_a_proposal_is_an_error():
+    """SU(3) with the reference's law and a delta that no proposal can be drawn
+    with: an error before any launch, the links unchanged.  Without hits or
+    sweeps, with the symmetric law, or in U(1) and SU(2), the call runs."""
+    dims = (4, 4, 4, 4)
+    for storage in ("f64", "f32", "f32_rows"):
+        g = klft.GaugeField(4, 3, dims, storage).set_random_algebra(0.4, 3)
+        before = g.download()
+        p = klft.MetropolisParams(nHits=2, beta=5.5, delta=0.0, seed=5)
+        with pytest.raises(klft.KlftError, match="delta"):
+            klft.sweep_Metropolis(g, p, 0)
+        with pytest.raises(klft.KlftError, match="delta"):
+            klft.metropolis_run(g, p, 0, 3)
+        with pytest.raises(klft.KlftError, match="delta"):
+            g.set_random_sun(0.0, 7)
+        klft.metropolis_run(g, p, 0, 0)
+        klft.sweep_Metropolis(g, klft.MetropolisParams(nHits=0, beta=5.5, delta=0.0, seed=5), 0)
+        assert np.array_equal(g.download(), before)
+        g.set_proposal("symmetric")
+        assert klft.sweep_Metropolis(g, p, 0) > 0.99  # the identity, dS = 0 up to rounding
+        g.close()
+        b = klft.Batch([(1, dims, 2.0), (3, dims, 5.5)], storage)
+        with pytest.raises(klft.KlftError, match="delta"):
+            b.sweep(2, 0.0, 7, 0)
+        with pytest.raises(klft.KlftError, match="delta"):
+            b.run(2, 0.0, 7, 0, 2)
+        b.run(2, 0.0, 7, 0, 0)
+        b.close()
+        r = klft.PTBC(2, 3, dims, 5.5, 2, [0, 1, 2], [1.0, 0.5], storage)
+        with pytest.raises(klft.KlftError, match="delta"):
+            r.step(2, 0.0, 7, 0)
+        r.close()
+        for nc in (1, 2):
+            h = klft.GaugeField(4, nc, dims, storage).set_random_sun(0.0, 7)
+            klft.sweep_Metropolis(h, p, 0)
+            h.close()

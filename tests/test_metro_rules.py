@@ -41,3 +41,18 @@ def test_drawing_a_row_ends(rules, delta):
     not finite."""
     for seed in range(20):
         assert rules("rows_drawn", delta, seed, 50) == [[1, 0]]
+
+
+@pytest.mark.parametrize("fp64,smallest,largest", [(1, 2.0 ** -54, 2.0 ** 513), (0, 2.0 ** -25, 2.0 ** 65)])
+def test_delta_without_a_proposal(rules, fp64, smallest, largest):
+    """Only a delta whose rows are next to never kept is refused: zero, below half
+    the smallest norm, above twice the largest (FP32 links: as a float).  One at the
+    limits keeps a row within some thousand draws."""
+    keep = [smallest, -smallest, largest, 0.1, 1.0, 1e-6, np.nan, np.inf, -np.inf] + ([] if fp64 else [1e300])
+    drop = [0.0, -0.0, 5e-324, smallest * (1 - 2.0 ** -22), largest * (1 + 2.0 ** -22), -2 * largest]
+    got = [bool(v[0]) for v in rules("rows_kept", fp64, *[float(d).hex() for d in keep + drop])]
+    assert got == [True] * len(keep) + [False] * len(drop)
+    if fp64:
+        for d in (smallest, -smallest):
+            assert rules("rows_drawn", d.hex(), 3, 20000)[0][1] == 0
+        assert rules("rows_drawn", "0", 3, 1000) == [[1000, 1]]
