@@ -111,11 +111,15 @@ int metropolis_variant(klft_field_t f, const klft_metropolis_params *p, bool tim
   const bool paired_one_round = 2 * ((f->g.Vh + 255) / 256) <= (long long)cu_count();
   const int dflt = ((f->storage == KLFT_STORAGE_F64 || paired_one_round) ? 13 : 12) +
                    (hits_in_parallel(f, p->nhits) ? 4 : 0);
-  // the symmetric SU(3) proposal runs in these kernels only
-  if (f->proposal == KLFT_PROPOSAL_SYMMETRIC && f->nc == 3) return dflt + 2;
   // KLFT_VARIANT="metropolis=v" forces a variant for every hit count
-  auto reference_law = [](int v) { return v != 14 && v != 15; };
   const int fv = forced_variant("metropolis");
+  // the symmetric SU(3) proposal runs in variants 14, 15, 18 and 19 only, those of
+  // 12, 13, 16 and 17
+  if (f->proposal == KLFT_PROPOSAL_SYMMETRIC && f->nc == 3) {
+    if (fv == 12 || fv == 13 || fv == 16 || fv == 17) return fv + 2;
+    return fv == 14 || fv == 15 || fv == 18 || fv == 19 ? fv : dflt + 2;
+  }
+  auto reference_law = [](int v) { return v != 14 && v != 15; };
   if (fv >= 0 && fv < kMetroVariants && reference_law(fv)) return fv;
   // the tuning key carries nHits: the best variant depends on the hit count
   const std::string kname = "metropolis_nhits_" + std::to_string(p->nhits);
