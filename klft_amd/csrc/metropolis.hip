@@ -64,25 +64,9 @@ static int launch_passes(klft_field_t f, void *links, int variant, int p0, int p
   return set_error(KLFT_E_ARG, "storage=%d unsupported", f->storage);
 }
 
-// Whether a pass of Vh sites runs faster with a link's hits in parallel
-// (metro_hits.hpp) than with site waves fed by staple waves.  The site-wave
-// kernel's pass costs one block's serial chain however few blocks there are;
-// the hit-parallel kernel's chain is four to six times shorter but spends up
-// to ten lanes on a site, so it wins until the sites fill the GPU.  Measured
-// ms per sweep in runs, nHits = 10, hit-parallel / site waves, around the
-// limits (sites of a pass per CU):
-//   SU(3)  16/CU (16^4) FP64 0.23 / 0.64, FP32 0.17 / 0.49; 81/CU (24^4) FP64
-//          0.68 / 0.71, FP32 0.44 / 0.50; with 1 hit 57/CU (22^4) 0.47 / 0.44
-//   SU(2)  16/CU FP64 0.32 / 0.52; 26/CU (18^4) 0.48 / 0.52, FP32 0.29 / 0.35;
-//          39/CU (20^4) 0.67 / 0.52
-//   U(1)   16/CU FP64 0.22 / 0.28; 26/CU 0.30 / 0.28, FP32 0.22 / 0.23; with 4
-//          hits 39/CU 0.16 / 0.19
-// and in 2D with fewer than 4 hits the site waves' chain is as short (U(1)
-// 32^2, 1 hit: 32 against 29 us).
-static bool hits_in_parallel(klft_field_t f, int nhits) {
-  if (f->nd == 2 && nhits < 4) return false;
-  const int per_cu = f->nc == 3 ? (nhits < 8 ? 48 : 81) : (f->nc == 2 ? 27 : (nhits < 5 ? 40 : 20));
-  return f->g.Vh <= (long long)per_cu * cu_count();
+static bool hits_in_parallel(klft_field_t f, const klft_metropolis_params *p) {
+  return klft_metro::hits_in_parallel(f->nd, f->nc, f->g.Vh, cu_count(), p->nhits, p->beta,
+                                      f->proposal == KLFT_PROPOSAL_SYMMETRIC);
 }
 
 // sweep variant for this field; tuning times one sweep of each variant on a
@@ -100,7 +84,7 @@ int metropolis_variant(klft_field_t f, const klft_metropolis_params *p, bool tim
   // numbers below kMetroVariants are not built (the tuner skips them), or run
   // the symmetric proposal (14, 15).
   // Untuned defaults: hits in parallel while the sites do not fill the GPU
-  // (hits_in_parallel), else site waves fed by staple waves, with the
+  // (metro_rules.hpp), else site waves fed by staple waves, with the
   // interleaved term order for FP64 links.  For FP32 links the interleaved
   // order's six loads in flight (196 VGPRs) leave room for one block per CU,
   // the upper-terms-first order (128 VGPRs) for two: the interleaved order
@@ -110,7 +94,7 @@ int metropolis_variant(klft_field_t f, const klft_metropolis_params *p, bool tim
   // alone, so that the FP32 results do not depend on which kernel runs.
   const bool paired_one_round = 2 * ((f->g.Vh + 255) / 256) <= (long long)cu_count();
   const int dflt = ((f->storage == KLFT_STORAGE_F64 || paired_one_round) ? 13 : 12) +
-                   (hits_in_parallel(f, p->nhits) ? 4 : 0);
+                   (hits_in_parallel(f, p) ? 4 : 0);
   // KLFT_VARIANT="metropolis=v" forces a variant for every hit count
   const int fv = forced_variant("metropolis");
   // the symmetric SU(3) proposal runs in variants 14, 15, 18 and 19 only, those of

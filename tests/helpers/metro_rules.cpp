@@ -35,5 +35,10 @@ int main(int argc, char **argv) {
       printf("%d\n", (int)klft_metro::rows_kept(strtod(argv[i], nullptr), atoi(argv[2]) != 0));
     return 0;
   }
+  if (!strcmp(argv[1], "hits_in_parallel")) {  // nd nc Vh cus nhits beta symmetric
+    printf("%d\n", (int)klft_metro::hits_in_parallel(atoi(argv[2]), atoi(argv[3]), atoll(argv[4]), atoi(argv[5]),
+                                                     atoi(argv[6]), strtod(argv[7], nullptr), atoi(argv[8]) != 0));
+    return 0;
+  }
   return 1;
 }

@@ -56,3 +56,24 @@ def test_delta_without_a_proposal(rules, fp64, smallest, largest):
         for d in (smallest, -smallest):
             assert rules("rows_drawn", d.hex(), 3, 20000)[0][1] == 0
         assert rules("rows_drawn", "0", 3, 1000) == [[1000, 1]]
+
+
+# sites of a pass on 256 CUs: 16^4, 18^4, 20^4, 22^4, 24^4
+VH = {L: L ** 4 // 16 for L in (16, 18, 20, 22, 24, 26)}
+
+
+@pytest.mark.parametrize("nc,nhits,beta,law,largest", [
+    # SU(3): the limit falls with the acceptance
+    (3, 10, 6.0, 0, 24), (3, 10, 5.0, 0, 22), (3, 10, 4.0, 0, 20), (3, 10, 2.5, 0, 16), (3, 10, 0.5, 0, 16),
+    (3, 10, 6.0, 1, 18), (3, 4, 6.0, 0, 20), (3, 4, 4.0, 0, 18), (3, 4, 0.5, 0, 16), (3, 4, 6.0, 1, 18),
+    (3, 1, 6.0, 0, 20), (3, 1, 2.5, 0, 16), (3, 1, 6.0, 1, 16), (3, 10, "nan", 0, 16), (3, 10, -5.0, 0, 16),
+    # SU(2), U(1): the same limit for every beta
+    (2, 10, 2.3, 0, 18), (2, 10, 0.1, 1, 18), (1, 10, 2.0, 0, 16), (1, 4, 0.1, 0, 20)])
+def test_hits_in_parallel_up_to_the_measured_size(rules, nc, nhits, beta, law, largest):
+    """The largest 4D lattice whose sweep takes the hit-parallel kernel, by group,
+    hits, beta and law.  Smaller ones always do, but for short hit chains in 2D."""
+    for L, vh in VH.items():
+        assert bool(rules("hits_in_parallel", 4, nc, vh, 256, nhits, beta, law)[0][0]) == (L <= largest), L
+    assert rules("hits_in_parallel", 4, nc, 14 ** 4 // 16, 256, nhits, beta, law) == [[1]]
+    assert rules("hits_in_parallel", 2, nc, 256, 256, 3, beta, law) == [[0]]
+    assert rules("hits_in_parallel", 2, nc, 256, 256, 4, beta, law) == [[1]]
