@@ -302,6 +302,138 @@ __global__ __launch_bounds__(256) void k_convert(Links<RO, NC, CO> o, Links<RI, 
 }
 
 // ============================================================================
+// per-site results
+// ============================================================================
+// n doubles into pinned host memory: a launch beside the kernels before it starts
+// where a copy engine would be waited for (20 us)
+__global__ __launch_bounds__(256) void k_to_host(const double *__restrict__ src, double *__restrict__ dst, int n) {
+  const int i = 2 * (int)(blockIdx.x * 256 + threadIdx.x);
+  if (i + 1 < n)
+    *reinterpret_cast<double2 *>(dst + i) = *reinterpret_cast<const double2 *>(src + i);
+  else if (i < n)
+    dst[i] = src[i];
+}
+
+namespace {
+// Per-site results pass through pinned pieces, the host copying one while the
+// next one arrives: a copy into pageable memory is staged by the runtime, or
+// pins and unpins the caller's pages (16^4 200 us).  With the array kept on the
+// device, and one wait instead of two, a plaquette with its sites takes 26 us
+// instead of 47 (10 x 10 x 8), 56 instead of 67 (SU(2) 16^4), 658 instead of 808
+// (SU(3) 32^4).
+//
+// The pieces (at most 2 MiB) and the array (at most 64 MiB, else one per call)
+// are the library's, not a field's: fresh ones cost a field's first such call 300 us
+// at 16^4.  They grow with the largest field that asks, and go when the last field
+// is destroyed.  A call holds the lock from its array to the end of its copy.
+class SiteStage {
+ public:
+  void field_created() {
+    std::lock_guard<std::mutex> lk(mu_);
+    ++fields_;
+  }
+  void field_destroyed() {
+    std::lock_guard<std::mutex> lk(mu_);
+    if (--fields_ == 0) release();
+  }
+  // per_site[0..n) <- what `fill` writes into a device array of n doubles
+  template <class F>
+  int run(size_t n, double *per_site, F &&fill) {
+    std::lock_guard<std::mutex> lk(mu_);
+    const size_t bytes = n * sizeof(double);
+    if (bytes > kMost) {
+      double *p = nullptr;
+      KLFT_HIP(hipMalloc((void **)&p, bytes));
+      int rc = fill(p);
+      if (!rc) rc = copy_out(per_site, p, bytes);
+      (void)hipFree(p);
+      return rc;
+    }
+    if (bytes > cap_) {
+      if (dev_) (void)hipFree(dev_);  // no call uses it: each one waits for its copy
+      dev_ = nullptr;
+      cap_ = 0;
+      KLFT_HIP(hipMalloc((void **)&dev_, bytes));
+      cap_ = bytes;
+    }
+    const int rc = fill(dev_);
+    return rc ? rc : copy_out(per_site, dev_, bytes);
+  }
+
+ private:
+  static constexpr size_t kMost = (size_t)64 << 20, kPiece = (size_t)1 << 20;
+
+  void release() {
+    if (dev_) (void)hipFree(dev_);
+    if (pin_) (void)hipHostFree(pin_);
+    for (hipEvent_t &e : full_) {
+      if (e) (void)hipEventDestroy(e);
+      e = nullptr;
+    }
+    dev_ = nullptr;
+    pin_ = nullptr;
+    cap_ = piece_ = 0;
+  }
+  // two pieces of at least min(bytes, kPiece) each; false: no pinned memory left
+  bool pieces(size_t bytes) {
+    const size_t want = std::min(kPiece, (bytes + 4095) / 4096 * 4096);
+    if (want <= piece_) return true;
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    piece_ = 0;
+    hipError_t e = hipHostMalloc((void **)&pin_, 2 * want, hipHostMallocDefault);
+    for (hipEvent_t &ev : full_)
+      if (e == hipSuccess && !ev) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
+    if (e == hipSuccess) {
+      piece_ = want;
+      return true;
+    }
+    if (pin_) (void)hipHostFree(pin_);
+    pin_ = nullptr;
+    (void)hipGetLastError();
+    return false;
+  }
+  // from the device to pageable host memory on the library stream, complete on
+  // return
+  int copy_out(double *dst, const double *src, size_t bytes) {
+    if (!pieces(bytes)) {
+      KLFT_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, ki::stream()));
+      KLFT_HIP(hipStreamSynchronize(ki::stream()));
+      return KLFT_OK;
+    }
+    const size_t n = (bytes + piece_ - 1) / piece_;
+    auto size = [&](size_t i) { return std::min(piece_, bytes - i * piece_); };
+    for (size_t i = 0; i <= n; ++i) {
+      if (i < n) {
+        const int vals = (int)(size(i) / sizeof(double));
+        hipLaunchKernelGGL(k_to_host, dim3(ki::blocks_for((vals + 1) / 2, 256)), dim3(256), 0, ki::stream(),
+                           src + i * (piece_ / sizeof(double)),
+                           reinterpret_cast<double *>(pin_ + (i & 1) * piece_), vals);
+        KLFT_HIP(hipGetLastError());
+        if (i + 1 < n) KLFT_HIP(hipEventRecord(full_[i & 1], ki::stream()));
+      }
+      if (i > 0) {
+        if (i < n)
+          KLFT_HIP(hipEventSynchronize(full_[(i - 1) & 1]));
+        else
+          KLFT_HIP(hipStreamSynchronize(ki::stream()));
+        std::memcpy(reinterpret_cast<char *>(dst) + (i - 1) * piece_, pin_ + ((i - 1) & 1) * piece_, size(i - 1));
+      }
+    }
+    return KLFT_OK;
+  }
+
+  std::mutex mu_;
+  int fields_ = 0;
+  double *dev_ = nullptr;
+  size_t cap_ = 0, piece_ = 0;
+  unsigned char *pin_ = nullptr;
+  hipEvent_t full_[2] = {nullptr, nullptr};
+};
+SiteStage g_sites;
+}  // namespace
+
+// ============================================================================
 // field lifecycle
 // ============================================================================
 extern "C" int klft_field_create(int nd, int nc, const int *dims, int storage, klft_field_t *out) {
@@ -359,14 +491,14 @@ extern "C" int klft_field_create(int nd, int nc, const int *dims, int storage, k
   // and here one of the set_* calls or an upload gives the start
   if (e == hipSuccess) e = hipMemsetAsync(f->links, 0, f->link_bytes, ki::stream());
   if (e == hipSuccess) e = hipStreamSynchronize(ki::stream());
-  const size_t sites = f->g.V <= ki::kPinWithResult ? (size_t)f->g.V : 0;
-  if (e == hipSuccess) e = hipHostMalloc((void **)&f->host_result, (16 + sites) * sizeof(double), hipHostMallocDefault);
+  if (e == hipSuccess) e = hipHostMalloc((void **)&f->host_result, 16 * sizeof(double), hipHostMallocDefault);
   if (e != hipSuccess) {
     (void)hipFree(w);
     (void)hipFree(f->links);
     delete f;
     return ki::hip_fail(e, "workspace init");
   }
+  g_sites.field_created();
   *out = f;
   return KLFT_OK;
 }
@@ -379,69 +511,9 @@ extern "C" int klft_field_destroy(klft_field_t f) {
   if (f->host_result) (void)hipHostFree(f->host_result);
   if (f->run_counters) (void)hipFree(f->run_counters);
   if (f->meas_ws) (void)hipFree(f->meas_ws);
-  if (f->pin) (void)hipHostFree(f->pin);
-  for (hipEvent_t e : f->pin_full)
-    if (e) (void)hipEventDestroy(e);
   f->links = nullptr;
   delete f;
-  return KLFT_OK;
-}
-
-// n doubles into pinned host memory: a launch beside the kernels before it starts
-// where a copy engine would be waited for (20 us)
-__global__ __launch_bounds__(256) void k_to_host(const double *__restrict__ src, double *__restrict__ dst, int n) {
-  const int i = 2 * (int)(blockIdx.x * 256 + threadIdx.x);
-  if (i + 1 < n)
-    *reinterpret_cast<double2 *>(dst + i) = *reinterpret_cast<const double2 *>(src + i);
-  else if (i < n)
-    dst[i] = src[i];
-}
-
-// Per-site results pass through pinned pieces, the host copying one while the
-// next one arrives: a copy into pageable memory is staged by the runtime, or
-// pins and unpins the caller's pages (16^4 200 us).  With the array kept on the
-// device, and one wait instead of two, a plaquette with its sites takes 26 us
-// instead of 47 (10 x 10 x 8), 56 instead of 67 (SU(2) 16^4), 658 instead of 808
-// (SU(3) 32^4).
-int klft_internal::copy_out(klft_field_t f, double *dst, const double *src, size_t nvals) {
-  const size_t bytes = nvals * sizeof(double);
-  const size_t piece = std::min(kPinBytes, (sizeof(double) * (size_t)f->g.V + 4095) / 4096 * 4096);
-  unsigned char *pin = f->pin;
-  if (f->g.V <= kPinWithResult) {
-    pin = reinterpret_cast<unsigned char *>(f->host_result + 16);
-  } else if (!pin) {
-    hipError_t e = hipHostMalloc((void **)&f->pin, 2 * piece, hipHostMallocDefault);
-    for (hipEvent_t &ev : f->pin_full)
-      if (e == hipSuccess && !ev) e = hipEventCreateWithFlags(&ev, hipEventDisableTiming);
-    if (e != hipSuccess) {  // no pinned memory left: the plain copy
-      if (f->pin) (void)hipHostFree(f->pin);
-      f->pin = nullptr;
-      (void)hipGetLastError();
-      KLFT_HIP(hipMemcpyAsync(dst, src, bytes, hipMemcpyDeviceToHost, stream()));
-      KLFT_HIP(hipStreamSynchronize(stream()));
-      return KLFT_OK;
-    }
-    pin = f->pin;
-  }
-  const size_t n = (bytes + piece - 1) / piece;
-  auto size = [&](size_t i) { return std::min(piece, bytes - i * piece); };
-  for (size_t i = 0; i <= n; ++i) {
-    if (i < n) {
-      const int vals = (int)(size(i) / sizeof(double));
-      hipLaunchKernelGGL(k_to_host, dim3(blocks_for((vals + 1) / 2, 256)), dim3(256), 0, stream(),
-                         static_cast<const double *>(src) + i * (piece / sizeof(double)),
-                         reinterpret_cast<double *>(pin + (i & 1) * piece), vals);
-      KLFT_HIP(hipGetLastError());
-      if (i + 1 < n) KLFT_HIP(hipEventRecord(f->pin_full[i & 1], stream()));
-    }
-    if (i > 0) {
-      if (i < n)
-        KLFT_HIP(hipEventSynchronize(f->pin_full[(i - 1) & 1]));
-      else
-        KLFT_HIP(hipStreamSynchronize(stream()));
-      std::memcpy(reinterpret_cast<char *>(dst) + (i - 1) * piece, pin + ((i - 1) & 1) * piece, size(i - 1));
-    }
-  }
+  g_sites.field_destroyed();
   return KLFT_OK;
 }
 
@@ -769,20 +841,19 @@ extern "C" int klft_plaquette(klft_field_t f, int normalize, double *out, double
   int rc = ki::check_field(f);
   if (rc) return rc;
   if (!out) return ki::set_error(KLFT_E_ARG, "null output");
-  void *dps = nullptr;
-  if (per_site) {
-    rc = ki::meas_workspace(f, sizeof(double) * f->g.V, &dps);
-    if (rc) return rc;
-  }
-  rc = ki::plaquette_raw(f, 0, static_cast<double *>(dps));
   double sum = 0.0;
-  if (!rc && per_site) {
-    // the sum travels ahead of the sites, with one wait for both
-    KLFT_HIP(hipMemcpyAsync(f->host_result, f->result, sizeof(double), hipMemcpyDeviceToHost, ki::stream()));
-    rc = ki::copy_out(f, per_site, static_cast<double *>(dps), (size_t)f->g.V);
+  if (per_site) {
+    rc = g_sites.run((size_t)f->g.V, per_site, [&](double *dps) -> int {
+      const int prc = ki::plaquette_raw(f, 0, dps);
+      if (prc) return prc;
+      // the sum travels ahead of the sites, with one wait for both
+      KLFT_HIP(hipMemcpyAsync(f->host_result, f->result, sizeof(double), hipMemcpyDeviceToHost, ki::stream()));
+      return KLFT_OK;
+    });
     sum = f->host_result[0];
-  } else if (!rc) {
-    rc = ki::read_results(f, 0, 1, &sum);
+  } else {
+    rc = ki::plaquette_raw(f, 0, nullptr);
+    if (!rc) rc = ki::read_results(f, 0, 1, &sum);
   }
   if (rc) return rc;
   if (normalize) {  // GaugePlaquette.hpp:125-132

@@ -30,7 +30,7 @@ struct klft_field_s {
   unsigned int *ticket = nullptr;
   double *result = nullptr;  // 16 doubles
   unsigned long long *counter = nullptr;  // kCounterRows rows of kCounterCols counters
-  double *host_result = nullptr;          // pinned, 16 doubles (and a small field's sites)
+  double *host_result = nullptr;          // pinned, 16 doubles
   // acceptance counters of klft_metropolis_run, kCounterRows rows of one per
   // sweep (grown on demand, kept until the field is destroyed)
   unsigned long long *run_counters = nullptr;
@@ -38,10 +38,6 @@ struct klft_field_s {
   // measurement workspace (Wilson-loop partials, outputs, extents; grown on
   // demand, kept until the field is destroyed)
   void *meas_ws = nullptr;
-  // two pinned pieces of at most kPinBytes that per-site results pass through, and the
-  // events that say when each is full (allocated at the first such call)
-  unsigned char *pin = nullptr;
-  hipEvent_t pin_full[2] = {nullptr, nullptr};
   size_t meas_capacity = 0;
   int proposal = KLFT_PROPOSAL_REFERENCE;  // SU(3) Metropolis proposal law
 };
@@ -79,12 +75,6 @@ kd::Geom make_geom(int nd, const int *dims);
 // the field's measurement workspace, at least `bytes` long (grown on demand;
 // growing synchronises the library stream before the old buffer is freed)
 int meas_workspace(klft_field_t f, size_t bytes, void **out);
-constexpr size_t kPinBytes = (size_t)1 << 20;
-// fields of at most this many sites keep them behind host_result
-constexpr long long kPinWithResult = 8192;
-// n doubles from the device to pageable host memory on the library stream,
-// complete on return
-int copy_out(klft_field_t f, double *dst, const double *src, size_t n);
 // enqueue-only helpers (no host synchronisation)
 int plaquette_raw(klft_field_t f, int slot, double *dev_per_site);  // sum into f->result[slot]
 int read_results(klft_field_t f, int first, int n, double *out);    // synchronises
