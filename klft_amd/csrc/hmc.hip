@@ -339,7 +339,12 @@ int enqueue_refresh(klft_hmc_t h, uint64_t traj, int slot) {
 // Directions per thread of k_step_dirs (1: a thread per link, k_md_step and
 // k_force).
 // Four dimensions: FP64 SU(3) takes two (746 against 787 us with one and 1300
-// with four at 32^4; 26.6, 33.6 and 59.7 at 12^4).  The others take all four once
+// with four at 32^4; 25.0, 33.6 and 58.6 at 12^4).  SU(3) with one block of
+// 17 to 64 sites per sublattice takes one, as a step lasts as long as one thread
+// there (FP64 4^3 x 8 14.0 against 15.5 us with two, 4^2 x 8^2 14.4 against 15.9, two
+// rows 11.8 against 13.9 and 11.9 against 14.0; above, 8^4 FP64 17.4 against 16.6;
+// below, where a thread per link runs short waves, 4^4 15.2 against 15.4 and 2^4
+// 23.1 against 14.7).  The others take all four once
 // the waves of two would wait for one another: U(1) and SU(2) from a wave per
 // SIMD on (SU(2) FP64 16^4 17.3 against 18.4 us, 12^4 14.1 against 13.8, 8^4 10.6
 // against 9.0; U(1) 32^4 54 against 65), FP32 SU(3), with two waves per SIMD at
@@ -350,6 +355,7 @@ int enqueue_refresh(klft_hmc_t h, uint64_t traj, int slot) {
 // direction, 64^2 8.7 against 6.9; 32^3 23.1 against 28.7).
 int directions_per_thread(const klft_field_s *f, bool streams) {
   if (f->nd < 4) return f->nc == 3 && f->g.V < 64 * 256 ? 1 : f->nd;
+  if (f->nc == 3 && f->g.Vh > 16 && f->g.Vh <= 64) return 1;
   if (f->nc == 3) return f->storage == KLFT_STORAGE_F64 || !streams ? 2 : 4;
   return f->g.V < 64 * 1024 ? 2 : 4;
 }

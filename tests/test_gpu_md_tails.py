@@ -85,3 +85,20 @@ def test_short_blocks_take_no_longer(monkeypatch, storage):
         h.close()
         g.close()
     assert t[0] < 1.25 * t[1], t
+
+
+def test_small_lattices_take_a_thread_per_link(monkeypatch):
+    """The default rule in SU(3), below, inside and above 17 to 64 sites of a
+    sublattice: the step's results are those of the variant it stands for."""
+    for dims, md, force in (((4, 4, 4, 4), 3, 6), ((4, 4, 6, 4), 1, 4), ((4, 4, 8, 8), 1, 4), ((4, 4, 10, 8), 3, 6)):
+        out = []
+        for v in ("x=0", f"md_step={md},force={force}"):
+            monkeypatch.setenv("KLFT_VARIANT", v)
+            g = klft.GaugeField(4, 3, dims, "f64").set_random_algebra(0.4, 7)
+            h = klft.HMC(g, beta=6.0, tau=0.2, nsteps=4, seed=3)
+            h.refresh_momenta(0)
+            h.integrate()
+            out.append((g.download(), h.momenta()))
+            h.close()
+            g.close()
+        assert np.array_equal(out[0][0], out[1][0]) and np.array_equal(out[0][1], out[1][1])
