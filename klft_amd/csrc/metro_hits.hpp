@@ -83,12 +83,11 @@ __device__ __forceinline__ void wave_lds_fence() {
 
 // The pass for positions t0 .. t0 + 64 / G - 1 of the sublattice, by a block
 // of W waves; returns the lane's accepted hits.  `lds`: 64 / G regions of
-// hit_stride reals.  DEFECT, SYM as in ws_pass.
-template <typename R, int NC, bool COMP, int ND, int W, bool ILV, bool DEFECT, bool SYM>
+// hit_stride reals.  SYM as in ws_pass.
+template <typename R, int NC, bool COMP, int ND, int W, bool ILV, bool SYM>
 __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, const Geom &g, int pass,
                                                   long long t0, int G, int nhits, R beta_nc, R delta, uint64_t seed,
-                                                  uint32_t sweep, uint32_t chain, int *visit, const Defect &d, R c,
-                                                  R *lds) {
+                                                  uint32_t sweep, uint32_t chain, int *visit, R *lds) {
   using SL = HitSlots<ND>;
   constexpr int NM = NC * NC, RS = hit_record<NC>();
   constexpr int NIT = SL::NU + SL::NL + 2 * ND;  // items of a site: products and link copies
@@ -116,7 +115,6 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
   };
   R *rec = region + 2 * (SL::N * NM | 1) + w * G * RS;  // the wave's proposal records
   uint32_t site = 0, s = 0;
-  R cown = R(1);  // the defect's factor on U_0(x)
   // neighbour offsets in 32 bits (fields hold < 2^32 sites), picked by value: a
   // select over an indexed array would put it in scratch
   uint32_t p0 = 0, p1 = 0, p2 = 0, p3 = 0, m0 = 0, m1 = 0, m2 = 0, m3 = 0;
@@ -127,7 +125,6 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
     sub_coords<ND>(g, pass, t, x);
     site = (uint32_t)lex_index<ND>(g, x);
     if (visit && e == 0 && w == 0) visit[site] = pass;
-    if constexpr (DEFECT) cown = on_defect<ND>(g, d, x, 0) ? c : R(1);
     const Nbr<ND> nb = make_nbr<ND>(g, x, (long long)pass * g.Vh + t);
     s = (uint32_t)nb.s;
     p0 = (uint32_t)nb.dp[0];
@@ -146,20 +143,9 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
   auto pick = [](int k, uint32_t v0, uint32_t v1, uint32_t v2, uint32_t v3) {
     return k < 0 ? 0u : (k == 0 ? v0 : (k == 1 ? v1 : (k == 2 ? v2 : v3)));
   };
-  // the link in direction dir at x + e_dp - e_dm (-1: none), defect-scaled if asked
-  auto link = [&](int dp, int dm, int dir, bool scaled) -> Mat<R, NC> {
-    Mat<R, NC> l = f.load((long long)(s + pick(dp, p0, p1, p2, p3) + pick(dm, m0, m1, m2, m3)), dir);
-    if constexpr (DEFECT) {
-      int y[ND];
-      shifted<ND>(g, x, dp, 1, dm, -1, y);
-      if (scaled && on_defect<ND>(g, d, y, dir)) {
-#pragma unroll
-        for (int i = 0; i < NC; ++i)
-#pragma unroll
-          for (int j = 0; j < NC; ++j) l.m[i][j] = scale(c, l.m[i][j]);
-      }
-    }
-    return l;
+  // the link in direction dir at x + e_dp - e_dm (-1: none)
+  auto link = [&](int dp, int dm, int dir) -> Mat<R, NC> {
+    return f.load((long long)(s + pick(dp, p0, p1, p2, p3) + pick(dm, m0, m1, m2, m3)), dir);
   };
   // items: the upper products, one link copy, the lower products, the other
   // copies (with ten lanes a wave's round holds one kind of product)
@@ -177,19 +163,19 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
           }
         }
         const int nu = j < mu ? j : j + 1;
-        const Mat<R, NC> ia = link(mu, -1, nu, true), ib = link(nu, -1, mu, true);
+        const Mat<R, NC> ia = link(mu, -1, nu), ib = link(nu, -1, mu);
         put(it, mul_ad(ia, ib));
       } else if (it > SL::NU && it <= SL::NU + SL::NL) {
         const int l = it - SL::NU - 1;
         const int mu = l / (ND - 1), j = l % (ND - 1);
         const int nu = j < mu ? j : j + 1;
-        const Mat<R, NC> ia = link(mu, nu, nu, true), ib = link(-1, nu, mu, true);
+        const Mat<R, NC> ia = link(mu, nu, nu), ib = link(-1, nu, mu);
         put(SL::NU + l, mul_dd(ia, ib));
       } else {
         const int k = it == SL::NU ? 0 : it - SL::NU - SL::NL;  // 0 .. 2 ND - 1
         const bool own = k < ND;
         const int dir = own ? k : k - ND;
-        put((own ? SL::U : SL::C) + dir, link(-1, own ? -1 : dir, dir, !own));
+        put((own ? SL::U : SL::C) + dir, link(-1, own ? -1 : dir, dir));
       }
     }
   }
@@ -205,8 +191,6 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
 #pragma unroll 1
   for (int mu = w; mu < ND; mu += W) {
     const int mslot = SL::m_slot(mu);
-    R cl = R(1);
-    if constexpr (DEFECT) cl = mu == 0 ? cown : R(1);
     // NC <= 2: the even lanes of a site carry M, the odd ones U
     const bool odd = (e & 1) != 0;
     Mat<R, NC> X = zero<R, NC>();
@@ -235,12 +219,7 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
         auto up = [&](int j, cx<R> v) -> cx<R> {
           const int nu = j < mu ? j : j + 1, sl = SL::upper(mu, j);
 #pragma unroll
-          for (int k = 0; k < NC; ++k) {
-            cx<R> b = at(SL::U + nu, ej, k);
-            if constexpr (DEFECT)
-              if (nu == 0) b = scale(cown, b);
-            v = cfma_c(at(sl, ei, k), b, v);
-          }
+          for (int k = 0; k < NC; ++k) v = cfma_c(at(sl, ei, k), at(SL::U + nu, ej, k), v);
           __builtin_amdgcn_sched_barrier(0);
           return v;
         };
@@ -283,12 +262,7 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
           // its first product is the adjoint of direction mu - 1's with mu
           const int sl = SL::upper(mu - 1, mu - 1);
 #pragma unroll
-          for (int k = 0; k < NC; ++k) {
-            cx<R> b = at(SL::U + mu - 1, ej, k);
-            if constexpr (DEFECT)
-              if (mu == 1) b = scale(cown, b);
-            v = cfma_c(conj(at(sl, k, ei)), b, v);
-          }
+          for (int k = 0; k < NC; ++k) v = cfma_c(conj(at(sl, k, ei)), at(SL::U + mu - 1, ej, k), v);
         }
         wave_lds_fence();
         if (entry) at(mslot, ei, ej) = v;
@@ -327,7 +301,7 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
           for (int k = 0; k < RS; ++k) nxt[k] = rec[hq * RS + k];
           // the decision is lane 0's; both products with p are one instruction
           // stream, and only U is restored
-          const bool acc = active && metro_accept(cl * (-beta_nc * (retr_mul(p, X) - trM)), ua);
+          const bool acc = active && metro_accept(-beta_nc * (retr_mul(p, X) - trM), ua);
           if ((__ballot(acc) >> (gi * G)) & 1ull) {
             changed = true;
             if (e == 0) ++n;
@@ -353,7 +327,7 @@ __device__ __forceinline__ unsigned int hits_pass(const Links<R, NC, COMP> &f, c
         bool live = active && h0 + e < nhits;
 #pragma unroll 1
         for (;;) {
-          const bool acc = live && metro_accept(cl * (-beta_nc * (retr_mul(r, M) - trM)), u);
+          const bool acc = live && metro_accept(-beta_nc * (retr_mul(r, M) - trM), u);
           const unsigned long long any = __ballot(acc);
           if (!any) break;
           const unsigned int mine = active ? (unsigned int)(any >> gsh) & gmask : 0u;
@@ -456,8 +430,8 @@ __global__ __launch_bounds__(64 * W, (HitOcc<R, NC>::value)) void k_metropolis_h
     }
     lb >>= 1;
   }
-  const unsigned int n = hits_pass<R, NC, COMP, ND, W, ILV, false, SYM>(
-      f, g, pass, (long long)lb * (64 / G), G, nhits, beta_nc, delta, seed, sweep, chain, visit, Defect{}, R(1),
+  const unsigned int n = hits_pass<R, NC, COMP, ND, W, ILV, SYM>(
+      f, g, pass, (long long)lb * (64 / G), G, nhits, beta_nc, delta, seed, sweep, chain, visit,
       reinterpret_cast<R *>(hits_smem));
   hits_count<W>(n, red, nacc + (size_t)(blockIdx.x % kCounterRows) * nacc_row);
 }
