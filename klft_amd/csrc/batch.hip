@@ -98,8 +98,8 @@ __global__ __launch_bounds__(kB) void k_batch_pass(const ChainDev *__restrict__ 
 // all eight waves meet the same barriers.
 // FP32 chains and replicas with the upper-terms-first order fit two blocks
 // per CU (128 VGPRs: four waves per SIMD); the register allocator is asked
-// for that (the defect kernels then spill 12 / 24 registers, FP32 two-row /
-// full, and still gain: C5 FP32 917 -> 956 steps/s, two-row 961 -> 1122
+// for that (the defect kernels then spill 15 / 25 registers, FP32 two-row /
+// full, and still gain: 16 SU(3) 16^4 replicas FP32 917 -> 956 steps/s, two-row 961 -> 1122
 // with their passes paired)
 template <typename R, bool COMP, bool DEFECT, bool ILV = false>
 __global__ __launch_bounds__(klft_metro::kWsBlock, (sizeof(R) == 4 && !ILV) ? 4 : 2) void k_batch_ws(

@@ -224,11 +224,29 @@ __device__ __forceinline__ unsigned long long ws_pass(const Links<R, NC, COMP> &
   auto build = [&](int sg, int defer, unsigned umask, unsigned lmask, Mat<R, NC> *keep) -> Mat<R, NC> {
     Mat<R, NC> acc = zero<R, NC>();
     const long long s_xp = idx_shift<ND>(g, x, sg, 1, -1, 0);
-    // the link at x + s1 e_m1 + s2 e_m2 in direction dir, defect-scaled
+    // The link at x + s1 e_m1 + s2 e_m2 in direction dir, defect-scaled.  The
+    // coordinates are needed for direction 0 alone; formed for every load and kept
+    // for the test after it, they cost FP32 SU(3) spills (29 registers instead of 25;
+    // a step of 16 replicas of 16^4 with one hit 885 -> 862 us).  FP64 links, where the
+    // registers suffice, form them (with the branch up to 4 % slower in U(1)).
     auto ld = [&](int m1, int s1, int m2, int s2, int dir) -> Mat<R, NC> {
-      int y[ND];
-      shifted<ND>(g, x, m1, s1, m2, s2, y);
-      return load_at<R, NC, COMP, ND, true>(f, g, y, dir, d, c);
+      if constexpr (sizeof(R) == 8) {
+        int y[ND];
+        shifted<ND>(g, x, m1, s1, m2, s2, y);
+        return load_at<R, NC, COMP, ND, true>(f, g, y, dir, d, c);
+      }
+      Mat<R, NC> u = f.load(m1 < 0 && m2 < 0 ? s : idx_shift<ND>(g, x, m1, s1, m2, s2), dir);
+      if (dir == 0) {
+        int y[ND];
+        shifted<ND>(g, x, m1, s1, m2, s2, y);
+        if (on_defect<ND>(g, d, y, 0)) {
+#pragma unroll
+          for (int i = 0; i < NC; ++i)
+#pragma unroll
+            for (int j = 0; j < NC; ++j) u.m[i][j] = scale(c, u.m[i][j]);
+        }
+      }
+      return u;
     };
     auto upper = [&](int j) {
       const int nu = j < sg ? j : j + 1;
