@@ -62,7 +62,8 @@ int klft_field_info(klft_field_t f, int *nd, int *nc, int *dims, int *storage);
 /* deviceGaugeField(L.., identitySUN<Nc>()) cold start (GaugeField.hpp:47-52, :80-93) */
 int klft_field_set_identity(klft_field_t f);
 /* deviceGaugeField(L.., rng, delta): every link a randSUN(delta) proposal
- * (GaugeField.hpp:55-60, :96-112), drawn from the keyed stream (tag 5). */
+ * (GaugeField.hpp:55-60, :96-112), drawn from the keyed stream (tag 5).  SU(3): a
+ * delta of 0, or one too small or too large for a row, is KLFT_E_ARG (below). */
 int klft_field_set_random_sun(klft_field_t f, double delta, uint64_t seed);
 /* U = exp(i eps Q), Q = sum_a h_a T_a / 2, h_a ~ N(0,1) keyed (seed, site, mu);
  * computed in FP64 and rounded to the field's storage. */

@@ -1017,7 +1017,7 @@ extern "C" int klft_staple_field(klft_field_t f, klft_field_t out) {
 // kWave: D moves between lanes, and a wave holds whole columns; else through LDS, in
 // two buffers (kLds2, a barrier a step) or one where two do not fit (kLds1).
 //
-// Bound by the vector unit, 216 FMAs for D and 36 for the trace of SU(3), with the
+// Bound by the vector unit, 216 FMAs for D and 18 for the trace of SU(3), with the
 // lane moves and 30 instructions of the wave's sum beside them: 64 loops of three
 // planes at 32^4 FP64 2.50 ms, their FP64 instructions alone 1.8 (FP32 1.28 ms).
 // With the thread at x loading U_nu(x+L mu+(T-1) nu) at each step, the

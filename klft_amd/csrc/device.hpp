@@ -1038,9 +1038,10 @@ __device__ __forceinline__ void rand_sun(klft_rng::Stream& s, R delta, Mat<R, 3>
 // computed up front.  The blocks are independent, so their rounds interleave
 // instead of forming one long dependent chain (a pass has one wave per SIMD
 // at 32^4, so nothing else hides that latency).  The SU(3) proposal's
-// rejection loops (SUN.hpp:198-233) repeat only when a norm is below 2^-53;
-// then the hit is redrawn by the looping rand_sun above from the start of the
-// same stream, which gives the same values, so the outcome is identical.
+// rejection loops (SUN.hpp:198-233) repeat only when a norm is below 2^-53
+// (FP32: 2^-24); FP32 then redraws the hit by the looping rand_sun above from the
+// start of the same stream, which gives the same values, and FP64 goes on row by
+// row (propose), so the outcome is identical.
 // ---------------------------------------------------------------------------
 template <typename R>
 struct DrawWords {  // stream words per uniform

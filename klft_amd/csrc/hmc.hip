@@ -133,8 +133,9 @@ __device__ __forceinline__ void store_stream(R *p, R v) {
 // still read it; the arithmetic is that of k_force followed by
 // k_update_gauge, so the result is the same.  One thread per link as in
 // k_force: a block holds one 64-site chunk, wave w taking direction w.  For the
-// SU(3) lattices in two and three dimensions that leave most CUs without a wave
-// (links_per_thread); the others take k_step_dirs.
+// SU(3) lattices where a step lasts as long as one thread (directions_per_thread);
+// the others take k_step_dirs.  Past the caches (NT) by request and in tuning only:
+// the rule's lattices fit them.
 template <typename R, int NC, bool COMP, int ND, bool NT>
 __global__ __launch_bounds__(256) void k_md_step(Links<R, NC, COMP> src, Links<R, NC, COMP> dst, R *P, Geom g,
                                                   R coef, R dtp, R dtu) {
@@ -173,9 +174,9 @@ __global__ __launch_bounds__(256) void k_md_step(Links<R, NC, COMP> src, Links<R
 // bytes in flight, and nearly each one waits for the memory-side cache or HBM, so
 // the time goes with the number of link loads, 19 a link with a thread per
 // link, 15 with two directions per thread, 11 with four (staples_of).
-// SU(3) 28x24x20x32 FP32 170 -> 145 us per step, 32^4 FP32 454 -> 345,
-// FP64 (two directions: four need 488 registers, one wave per SIMD) 860 -> 746,
-// SU(2) 16^4 FP64 32 -> 17.
+// SU(3) 28x24x20x32 FP32 170 -> 145 us per step, 32^4 FP32 454 -> 340,
+// FP64 (two directions, 256 registers and 8 spilled, 14 in the force; four need 488,
+// one wave per SIMD) 860 -> 731, SU(2) 16^4 FP64 32 -> 17.
 // With ND directions the next term's links are in flight while a term is
 // multiplied; with two, twice the waves do the same and the registers
 // that takes would cost one (SU(3) FP64 32^4 950 us).

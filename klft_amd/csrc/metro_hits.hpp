@@ -14,8 +14,9 @@
 //
 // SU(3): all G hits are judged at once against the same M.  The first accepted
 // one is final (and so are the rejected ones before it); M becomes M r and the
-// hits after it are judged again, so a link costs 1 + (accepted hits) rounds
-// (under 1 % of the reference's SU(3) proposals are accepted).  U(1) and SU(2):
+// hits after it are judged again, so a link costs 1 + (accepted hits) rounds (of
+// the reference's SU(3) proposals 3 % are accepted at beta = 6; hits_in_parallel
+// keeps this kernel from sizes where many rounds lose).  U(1) and SU(2):
 // most hits are accepted, so the lanes step through the hits, the proposals
 // handed over through LDS, the even lanes multiplying M and the odd ones U.
 //
